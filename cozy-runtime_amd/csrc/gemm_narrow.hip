@@ -51,17 +51,23 @@ __device__ __forceinline__ void w4_levels(const float* codebook, float (&book)[1
     for (int c = 0; c < 16; ++c) book[c] = codebook != nullptr ? codebook[c] : static_cast<float>(c - 8);
 }
 
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t whole_view(const void* p, int64_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes > 0x7fffffff ? 0x7fffffff : static_cast<int>(bytes), 0x00020000);
+}
+
+// The int8 level of a codebook level at group scale e, as a byte.
+__device__ __forceinline__ uint32_t w4_level(float level, float e) {
+    float r = __builtin_rintf(level * e);  // torch.round: half to even
+    r = __builtin_isnan(r) ? 0.0f : fminf(fmaxf(r, -127.0f), 127.0f);
+    return static_cast<uint8_t>(static_cast<int>(r));
+}
+
 // T[b][c] for b = the calling thread's index (256 threads), as 16 bytes at table + 16·b.
 __device__ __forceinline__ void w4_table_row(const float (&book)[16], uint32_t* table, int b) {
     const float e = e4m3_value(static_cast<uint32_t>(b));
     uint32_t words[4] = {0, 0, 0, 0};
 #pragma unroll
-    for (int c = 0; c < 16; ++c) {
-        const float level = book[c];
-        float r = __builtin_rintf(level * e);  // torch.round: half to even
-        r = __builtin_isnan(r) ? 0.0f : fminf(fmaxf(r, -127.0f), 127.0f);
-        words[c / 4] |= static_cast<uint32_t>(static_cast<uint8_t>(static_cast<int>(r))) << (8 * (c % 4));
-    }
+    for (int c = 0; c < 16; ++c) words[c / 4] |= w4_level(book[c], e) << (8 * (c % 4));
     *reinterpret_cast<uint4*>(table + 4 * b) = make_uint4(words[0], words[1], words[2], words[3]);
 }
 
@@ -81,8 +87,8 @@ __device__ __forceinline__ uint4 w4_unpack16(uint32_t c01, uint32_t c23, const u
         const uint32_t sel = spread & 0x07070707u;
         const uint32_t lo = __builtin_amdgcn_perm(t.y, t.x, sel);  // levels of codes 0..7
         const uint32_t hi = __builtin_amdgcn_perm(t.w, t.z, sel);  // levels of codes 8..15
-        const uint32_t m = ((spread >> 3) & 0x01010101u) * 0xffu;
-        return (hi & m) | (lo & ~m);
+        // Byte i of lo where the code's bit 3 is clear, else byte i of hi (selector 4 + i).
+        return __builtin_amdgcn_perm(hi, lo, ((spread >> 1) & 0x04040404u) | 0x03020100u);
     };
     uint32_t out[4];
 #pragma unroll
@@ -529,15 +535,8 @@ constexpr int kW4Rows = 4;       // weight rows a wave
 constexpr int kW4Batch = 2;      // 1 KiB code spans of each row in flight
 constexpr int kW4MaxK = 8192;    // activation rows a thread stages: K ≤ this
 constexpr int kW4Policy = 3;     // sc0 nt: each code byte is read once per call
-constexpr int kW4RowsMax = 16;   // rows the row-tile form takes (one MFMA's B columns)
-// 17..32 rows: the row-tile form with two 16-row activation blocks, for K ≤ 4096 (its
-// activation registers) and M·K ≤ 98304. Graph replays over weights past the MALL, µs narrow
-// tile / row tile, bit-equal: K=3072 N=12288 M=17 19.6 / 15.3, M=24 19.7 / 16.2, M=32 19.7 /
-// 17.7; K=4096 N=14336 M=20 25.1 / 22.5, M=32 25.1 / 26.2 (past the area rule); K=3072 N=3072
-// M=32 19.0 / 8.5.
-constexpr int kW4Rows2Max = 32;
-constexpr int kW4Rows2MaxK = 4096;
-constexpr int64_t kW4Rows2Area = 98304;
+constexpr int kW4RowsMax = 64;   // rows the row-tile form takes (one to four MFMAs' B columns)
+constexpr int kW4RowsK = 1024;   // past 32 rows, with K of this and more
 constexpr int kW4GemvRows = 2;   // rows the GEMV form takes
 constexpr uint32_t kFarW4 = 0x7fff0000u;  // a buffer offset past every resource here (reads 0)
 
@@ -674,157 +673,241 @@ __global__ __launch_bounds__(64 * kW4Waves) void w4a8_decode_kernel(
     }
 }
 
-// The w4a8.convrot linear for 3..32 quantized rows: one 16-row weight tile a workgroup, its K
-// split over kW4RWaves waves, on the plain v_mfma_i32_16x16x64_i8 (A = 16 weight rows, B = the
+// What four consecutive outputs of one row need after their sums: the row's scale, the weight
+// rows' scales and biases (bounded loads: zeros past M or N).
+struct Int8Epilogue {
+    float xs;
+    f32x4 ws;
+    i32x2 bias;
+};
+
+__device__ __forceinline__ Int8Epilogue int8_epilogue(const float* xs, const float* ws, const uint16_t* bias,
+                                                      int row, int n, int M, int N) {
+    Int8Epilogue e;
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(xs), 0, 4 * M, 0x00020000);
+    const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(ws), 0, 4 * N, 0x00020000);
+    e.xs = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, 4 * row, 0, 0));
+    e.ws = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(sr, 4 * n, 0, 0));
+    e.bias = i32x2{0, 0};
+    if (bias != nullptr) {
+        const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(bias), 0, 2 * N, 0x00020000);
+        e.bias = __builtin_bit_cast(i32x2, __builtin_amdgcn_raw_buffer_load_b64(br, 2 * n, 0, 0));
+    }
+    return e;
+}
+
+// Four consecutive outputs of one row by the int8 law (internal/int8_linear.py:445-448, then
+// :276): (acc·xs)·ws, cast, + bias in the output dtype.
+template <bool kOutHalf>
+__device__ __forceinline__ void int8_store4(i32x4 acc, const Int8Epilogue& e, bool biased, uint16_t* out) {
+    uint32_t o[2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float v = __fmul_rn(__fmul_rn(static_cast<float>(acc[i]), e.xs), e.ws[i]);
+        uint32_t h = ::cozyq::narrow<kOutHalf>(v);  // (this file's `narrow` launcher hides it)
+        const uint16_t b = static_cast<uint16_t>(static_cast<uint32_t>(e.bias[i / 2]) >> (16 * (i & 1)));
+        if (biased)
+            h = ::cozyq::narrow<kOutHalf>(__fadd_rn(widen<kOutHalf>(static_cast<uint16_t>(h)), widen<kOutHalf>(b)));
+        o[i / 2] = (i & 1) ? (o[i / 2] | (h << 16)) : h;
+    }
+    *reinterpret_cast<uint2*>(out) = make_uint2(o[0], o[1]);
+}
+
+// The w4a8.convrot linear for up to 64 quantized rows: kTiles 16-row weight tiles a workgroup, their
+// K split over kWaves waves, on the plain v_mfma_i32_16x16x64_i8 (A = 16 weight rows, B = the
 // activation rows, zero past M; kCols blocks of 16 of them, each A unpacked once for all).
 // Lane l (row r = l%16, part g = l/16) of a wave loads 16 contiguous code bytes of weight row r
 // per 128-code step t (codes 128t + 32g .. + 32: two groups, whose two scale bytes are adjacent)
 // and the same 32 activation elements of row r in two 16-byte pieces, so each of the step's two
-// MFMAs meets A and B on the same 16 k's; the 4 lanes of a row read 64 contiguous bytes. Every
-// load is issued before the level table is built; steps past a wave's share read zeros
-// (activation zeros make them add nothing). The waves' int32 partials meet in LDS (exact, in any
-// order), and the epilogue is the int8 law's, so the outputs equal every tile config's bit for
-// bit.
-constexpr int kW4RWaves = 4;
-
-template <bool kOutHalf, bool kBias, int kSteps, int kCols>
-__global__ __launch_bounds__(64 * kW4RWaves) void w4a8_rows_kernel(
+// MFMAs meets A and B on the same 16 k's; the 4 lanes of a row read 64 contiguous bytes. A pass
+// takes kWaves x kSteps steps, all its loads issued before any is used (the first pass's before
+// the level table is built); steps past a wave's share read zeros (activation zeros make them
+// add nothing). The waves' int32 partials meet in LDS (exact, in any order), and the epilogue is
+// the int8 law's, so the outputs equal every tile config's bit for bit.
+// Bound: half the time of K=3072 N=12288 M=16 (11.5 us; the 21.2 MB stream alone with everything
+// else taken out 6.1) is the unpack's VALU work (~90 instructions a step and wave) and the
+// activation reads through L2, neither of which overlaps the one burst of loads. A persistent form
+// (a workgroup a CU walking its tiles, the next tiles' codes in flight) measured 12.6 - 13.3 there.
+template <int kWaves, int kSteps, int kCols, int kTiles>
+__global__ __launch_bounds__(64 * kWaves) void w4a8_rows_kernel(
     const int8_t* q, const float* xs, const uint8_t* codes, W4 w4, const float* ws,
-    const uint16_t* bias, uint16_t* out, int M, int N, int K) {
+    const uint16_t* bias, uint16_t* out, int out_half, int M, int N, int K) {
     // (No pointer here is __restrict__: loads through restrict read-only arguments count as
     // invariant and may be sunk below later loads; these must stay in issue order.)
+    constexpr int kMakers = 64 * kWaves / 256;  // threads that build one level-table row
+    constexpr int kLevels = 16 / kMakers;       // levels each of them makes
+    constexpr int kBlocks = kCols * kTiles;     // 16x16 output blocks a workgroup
+    static_assert(kWaves % 4 == 0 && kWaves <= 16, "waves");
     __shared__ __attribute__((aligned(16))) uint32_t table[256 * 4];
-    __shared__ i32x4 part[kW4RWaves][kCols][64];
+    __shared__ i32x4 part[kWaves][kBlocks][64];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, g = lane >> 4;
-    const int n0 = blockIdx.x * 16;
+    const int n0 = blockIdx.x * (16 * kTiles);
     const int steps = K / 128;  // K % 256 == 0
-    const int t0 = wave * steps / kW4RWaves, t1 = (wave + 1) * steps / kW4RWaves;
 
-    // 0. The codebook's levels ahead of the streams: the table is built once they are issued,
-    //    and a wait for a load issued after them would wait for every one of them (in order).
-    float book[16];
-    w4_levels(w4.codebook, book);
-    asm volatile("" ::: "memory");
+    // 0. The epilogue's operands (wave b adds block b: tile b / kCols, columns b % kCols) and the
+    //    codebook's levels ahead of the streams: a wait for a load issued after them would wait
+    //    for every one of them (in order).
+    constexpr int kFinal = (kBlocks + kWaves - 1) / kWaves;  // blocks a wave adds at the end
+    Int8Epilogue epi[kFinal];
+#pragma unroll
+    for (int f = 0; f < kFinal; ++f) {
+        const int b = wave + f * kWaves;
+        if (b < kBlocks) epi[f] = int8_epilogue(xs, ws, bias, 16 * (b % kCols) + r, n0 + 16 * (b / kCols) + 4 * g, M, N);
+    }
+    const int first_level = kLevels * (tid & (kMakers - 1));
+    float book[kLevels];
+    if (w4.codebook != nullptr) {
+#pragma unroll
+        for (int c = 0; c < kLevels; ++c) book[c] = w4.codebook[first_level + c];
+    } else {
+#pragma unroll
+        for (int c = 0; c < kLevels; ++c) book[c] = static_cast<float>(first_level + c - 8);
+    }
+    fence();
 
-    // 1. The activation pieces: row 16c + r of each 16-row block c, elements 128t + 32g + 16h
-    //    .. + 16 (zeros past M or the wave's steps).
-    const __amdgpu_buffer_rsrc_t qr = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(q), 0, M * K, 0x00020000);
+    // Every load below is in bounds by itself: rows past N or M read the last row, steps past the
+    // wave's share its last one, and nothing uses what they bring. An address is a lane's row and
+    // part, the same for every step, plus the step's uniform offset: the address arithmetic and
+    // bounds of 24 loads, 600 instructions, were a third of a workgroup's.
+    const __amdgpu_buffer_rsrc_t qr = whole_view(q, static_cast<int64_t>(M) * K);
+    const __amdgpu_buffer_rsrc_t cr = whole_view(codes + static_cast<int64_t>(n0) * (K / 2), static_cast<int64_t>(N - n0) * (K / 2));
+    const __amdgpu_buffer_rsrc_t gr = whole_view(w4.group_scale + static_cast<int64_t>(n0) * (K / 16), static_cast<int64_t>(N - n0) * (K / 16));
+    uint32_t code_at[kTiles], scale_at[kTiles], x_at[kCols];
+#pragma unroll
+    for (int i = 0; i < kTiles; ++i) {
+        const int row = min(16 * i + r, N - 1 - n0);
+        code_at[i] = row * (K / 2) + 16 * g;
+        scale_at[i] = row * (K / 16) + 2 * g;
+    }
+#pragma unroll
+    for (int c = 0; c < kCols; ++c) x_at[c] = min(16 * c + r, M - 1) * K + 32 * g;
     i32x4 xb[kCols][kSteps][2];
+    uint4 cv[kTiles][kSteps];
+    uint32_t sv[kTiles][kSteps];
+    int t0, t1;
+    // One pass's loads: the wave's steps t0 .. t1 - 1 of the pass's, step by step, so that the
+    // first step's products wait for its own loads alone: the codes (16 bytes a lane,
+    // non-temporal), the lane's two group-scale bytes, and the activation pieces: row 16c + r of
+    // each 16-row block c, elements 128t + 32g + 16h .. + 16.
+    auto issue = [&](int pass) {
+        const int p0 = pass * (kWaves * kSteps), width = min(kWaves * kSteps, steps - p0);
+        t0 = p0 + wave * width / kWaves;
+        t1 = p0 + (wave + 1) * width / kWaves;
 #pragma unroll
-    for (int c = 0; c < kCols; ++c)
+        for (int j = 0; j < kSteps; ++j) {
+            const int t = min(t0 + j, max(t0, t1 - 1));  // t0 < steps: a pass has a step at least
 #pragma unroll
-        for (int j = 0; j < kSteps; ++j)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int t = t0 + j, row = 16 * c + r;
-                const uint32_t off = t < t1 && row < M ? static_cast<uint32_t>(row * K + 128 * t + 32 * g + 16 * h) : kFarW4;
-                xb[c][j][h] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(qr, off, 0, 0));
+            for (int i = 0; i < kTiles; ++i) {
+                cv[i][j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(cr, code_at[i], 64 * t, kW4Policy));
+                sv[i][j] = __builtin_amdgcn_raw_buffer_load_b16(gr, scale_at[i], 8 * t, 0);
             }
-    asm volatile("" ::: "memory");
-
-    // 2. The codes (16 bytes a lane a step, non-temporal) and the group scales.
-    const int64_t rows_bytes = static_cast<int64_t>(N - n0) * (K / 2);
-    const __amdgpu_buffer_rsrc_t cr = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(codes + static_cast<int64_t>(n0) * (K / 2)), 0,
-        rows_bytes > 0x7fffffff ? 0x7fffffff : static_cast<int>(rows_bytes), 0x00020000);
-    const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(w4.group_scale + static_cast<int64_t>(n0) * (K / 16)), 0,
-        static_cast<int>(static_cast<int64_t>(N - n0) * (K / 16)), 0x00020000);
-    uint4 cv[kSteps];
 #pragma unroll
-    for (int j = 0; j < kSteps; ++j) {
-        const int t = t0 + j;
-        const bool live = t < t1 && n0 + r < N;
-        cv[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
-            cr, live ? static_cast<uint32_t>(r * (K / 2) + 64 * t + 16 * g) : kFarW4, 0, kW4Policy));
-    }
-    // The group scales: one 16-byte load brings row r's scale bytes of two steps (8 a step, the
-    // four lane groups' pairs) where a 2-byte load a step brought a lane's own pair; the lane
-    // shifts its pair out at the product. Bytes of a dead step are never used (its activation
-    // reads zeros). Measured (graph replays, weights past the MALL): M = 16, K = 3072, N = 12288
-    // 12.6 -> 11.8 us; M = 4 10.7 -> 10.0.
-    constexpr int kPairs = (kSteps + 1) / 2;
-    uint4 sv[kPairs];
+            for (int c = 0; c < kCols; ++c)
 #pragma unroll
-    for (int u = 0; u < kPairs; ++u) {
-        const int t = t0 + 2 * u;
-        const bool live = t < t1 && n0 + r < N;
-        sv[u] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
-            gr, live ? static_cast<uint32_t>(r * (K / 16) + 8 * t) : kFarW4, 0, 0));
-    }
+                for (int h = 0; h < 2; ++h)
+                    xb[c][j][h] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(qr, x_at[c] + 16 * h, 128 * t, 0));
+            fence();
+        }
+    };
+    issue(0);
+    __builtin_amdgcn_sched_barrier(0);
 
-    // 3. The level table (row tid); a bare barrier (a full one would also wait for the loads).
-    w4_table_row(book, table, tid);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+    // The level table; a bare barrier (a full one would also wait for the loads).
+    {
+        const float e = __builtin_amdgcn_cvt_f32_fp8(tid / kMakers, 0);  // E4M3FN, NaN kept
+#pragma unroll
+        for (int c = 0; c < kLevels; c += 4) {
+            uint32_t word = w4_level(book[c], e);
+#pragma unroll
+            for (int i = 1; i < 4; ++i) word |= w4_level(book[c + i], e) << (8 * i);
+            table[4 * (tid / kMakers) + (first_level + c) / 4] = word;
+        }
+    }
+    fence();
+    wait_lgkmcnt0();
     __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    fence();
 
-    // 4. Products over the wave's steps.
-    i32x4 acc[kCols];
+    // Products over the wave's steps, pass by pass.
+    i32x4 acc[kTiles][kCols];
 #pragma unroll
-    for (int c = 0; c < kCols; ++c) acc[c] = i32x4{0, 0, 0, 0};
+    for (int i = 0; i < kTiles; ++i)
 #pragma unroll
-    for (int j = 0; j < kSteps; ++j) {
-        const uint4 s4 = sv[j / 2];
-        const uint32_t d = (j & 1) ? ((g >> 1) ? s4.w : s4.z) : ((g >> 1) ? s4.y : s4.x);
-        const uint32_t sb = (d >> (16 * (g & 1))) & 0xffffu;
-        const i32x4 l0 = __builtin_bit_cast(i32x4, w4_unpack16(cv[j].x, cv[j].y, table, sb & 0xffu));
-        const i32x4 l1 = __builtin_bit_cast(i32x4, w4_unpack16(cv[j].z, cv[j].w, table, sb >> 8));
+        for (int c = 0; c < kCols; ++c) acc[i][c] = i32x4{0, 0, 0, 0};
+    const int passes = (steps + kWaves * kSteps - 1) / (kWaves * kSteps);
+    for (int pass = 0; pass < passes; ++pass) {
+        if (pass != 0) issue(pass);
 #pragma unroll
-        for (int c = 0; c < kCols; ++c) {
-            acc[c] = mfma_i8(l0, xb[c][j][0], acc[c]);
-            acc[c] = mfma_i8(l1, xb[c][j][1], acc[c]);
+        for (int j = 0; j < kSteps; ++j) {
+            if (t0 + j >= t1) break;  // uniform
+#pragma unroll
+            for (int i = 0; i < kTiles; ++i) {
+                const uint32_t sb = sv[i][j];
+                const i32x4 l0 = __builtin_bit_cast(i32x4, w4_unpack16(cv[i][j].x, cv[i][j].y, table, sb & 0xffu));
+                const i32x4 l1 = __builtin_bit_cast(i32x4, w4_unpack16(cv[i][j].z, cv[i][j].w, table, sb >> 8));
+#pragma unroll
+                for (int c = 0; c < kCols; ++c) {
+                    acc[i][c] = mfma_i8(l0, xb[c][j][0], acc[i][c]);
+                    acc[i][c] = mfma_i8(l1, xb[c][j][1], acc[i][c]);
+                }
+            }
         }
     }
 
-    // 5. The waves' partials (lane l: activation row l%16, weight rows 4·(l/16) + 0..3), then
-    //    (acc·xs)·ws, cast, + bias in the output dtype (internal/int8_linear.py:445-448, :276).
+    // The waves' partials (lane l: activation row l%16, weight rows 4·(l/16) + 0..3) meet, then
+    // (acc·xs)·ws, cast, + bias in the output dtype (internal/int8_linear.py:445-448, :276).
 #pragma unroll
-    for (int c = 0; c < kCols; ++c) part[wave][c][lane] = acc[c];
+    for (int i = 0; i < kTiles; ++i)
+#pragma unroll
+        for (int c = 0; c < kCols; ++c) part[wave][i * kCols + c][lane] = acc[i][c];
     __syncthreads();
-    if (wave != 0) return;
-    const int n = n0 + 4 * g;
-    if (n >= N) return;  // N % 8 == 0: a lane's four rows are all in or all out
 #pragma unroll
-    for (int c = 0; c < kCols; ++c) {
+    for (int f = 0; f < kFinal; ++f) {
+        const int b = wave + f * kWaves;
+        const int row = 16 * (b % kCols) + r, n = n0 + 16 * (b / kCols) + 4 * g;
+        if (b >= kBlocks || row >= M || n >= N) continue;  // N % 8 == 0: a lane's four rows are all in or all out
+        i32x4 sum = part[0][b][lane];
 #pragma unroll
-        for (int w = 1; w < kW4RWaves; ++w) acc[c] += part[w][c][lane];
-        const int row = 16 * c + r;
-        if (row >= M) continue;
-        uint32_t o[2];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float v = __fmul_rn(__fmul_rn(static_cast<float>(acc[c][i]), xs[row]), ws[n + i]);
-            uint32_t h = ::cozyq::narrow<kOutHalf>(v);
-            if constexpr (kBias)
-                h = ::cozyq::narrow<kOutHalf>(__fadd_rn(widen<kOutHalf>(static_cast<uint16_t>(h)), widen<kOutHalf>(bias[n + i])));
-            o[i / 2] = (i & 1) ? (o[i / 2] | (h << 16)) : h;
-        }
-        *reinterpret_cast<uint2*>(out + static_cast<int64_t>(row) * N + n) = make_uint2(o[0], o[1]);
+        for (int v = 1; v < kWaves; ++v) sum += part[v][b][lane];
+        uint16_t* dst = out + static_cast<int64_t>(row) * N + n;
+        if (out_half)
+            int8_store4<true>(sum, epi[f], bias != nullptr, dst);
+        else
+            int8_store4<false>(sum, epi[f], bias != nullptr, dst);
     }
 }
 
-template <bool kOutHalf, bool kBias>
+template <int kCols>
 hipError_t launch_w4a8_rows(const int8_t* q, const float* xs, const uint8_t* codes, W4 w4, const float* ws,
-                            const void* bias, void* out, int M, int N, int K, hipStream_t s) {
-    const int blocks = (N + 15) / 16;
-    const int per_wave = (K / 128 + kW4RWaves - 1) / kW4RWaves;
+                            const void* bias, void* out, bool out_half, int M, int N, int K, hipStream_t s) {
     const auto* b = static_cast<const uint16_t*>(bias);
     auto* o = static_cast<uint16_t*>(out);
-    if (M > 16) {  // two 16-row activation blocks (the caller keeps K <= kW4Rows2MaxK)
-        if (per_wave <= 4)
-            w4a8_rows_kernel<kOutHalf, kBias, 4, 2><<<blocks, 64 * kW4RWaves, 0, s>>>(q, xs, codes, w4, ws, b, o, M, N, K);
-        else
-            w4a8_rows_kernel<kOutHalf, kBias, 8, 2><<<blocks, 64 * kW4RWaves, 0, s>>>(q, xs, codes, w4, ws, b, o, M, N, K);
-    } else if (per_wave <= 4)
-        w4a8_rows_kernel<kOutHalf, kBias, 4, 1><<<blocks, 64 * kW4RWaves, 0, s>>>(q, xs, codes, w4, ws, b, o, M, N, K);
-    else if (per_wave <= 8)
-        w4a8_rows_kernel<kOutHalf, kBias, 8, 1><<<blocks, 64 * kW4RWaves, 0, s>>>(q, xs, codes, w4, ws, b, o, M, N, K);
-    else
-        w4a8_rows_kernel<kOutHalf, kBias, 16, 1><<<blocks, 64 * kW4RWaves, 0, s>>>(q, xs, codes, w4, ws, b, o, M, N, K);
+    // Steps a wave a pass: as few in all, dead ones counted, as 1 .. 4 a pass allow, then the
+    // longest passes.
+    const int steps = K / 128;
+    int per = 1, least = steps;
+    for (int c = 1; c <= 4; ++c) {
+        const int total = (steps + 8 * c - 1) / (8 * c) * c;
+        if (total <= least) per = c, least = total;
+    }
+    // Tiles a workgroup: as many as leave one workgroup a CU, so that a level table and an
+    // activation piece serve all of a CU's tiles (K=4096 N=14336 M=16 one tile 17.3, four 14.4 us;
+    // M=64 28.0 and 21.0; K=2048 N=8192 M=16 6.6 and 6.0). Up to 8 rows there are few activation
+    // bytes to share and one tile a workgroup, three a CU, is faster (K=3072 N=12288 M=3 10.5
+    // and 9.2), but not past that (K=4096 N=14336 M=5 14.7 and 13.4).
+    const int tiles = (N + 15) / 16;
+    const int share = M <= 8 && tiles <= 768 ? 1 : min(4, (tiles + 255) / 256);
+#define COZYQ_GO(S, T) w4a8_rows_kernel<8, S, kCols, T><<<(N + 16 * T - 1) / (16 * T), 512, 0, s>>>(q, xs, codes, w4, ws, b, o, out_half, M, N, K)
+    if (share == 4) COZYQ_GO(1, 4);
+    else if (share == 3) COZYQ_GO(2, 3);
+    else if (share == 2) COZYQ_GO(2, 2);
+    else if (per == 1) COZYQ_GO(1, 1);
+    else if (per == 2) COZYQ_GO(2, 1);
+    else if (per == 3) COZYQ_GO(3, 1);
+    else COZYQ_GO(4, 1);
+#undef COZYQ_GO
     return hipGetLastError();
 }
 
@@ -835,6 +918,7 @@ hipError_t launch_w4a8_rows(const int8_t* q, const float* xs, const uint8_t* cod
 // same k's of each activation row, zeros past K, M or N. The waves' int32 partials meet in LDS
 // and the epilogue is the int8 law's, so the outputs equal every tile config's bit for bit.
 constexpr int kI8RowsMaxK = 4096;
+constexpr int kW4RWaves = 4;  // waves a workgroup
 
 template <bool kOutHalf, bool kBias, int kSteps, int kCols>
 __global__ __launch_bounds__(64 * kW4RWaves) void int8_rows_kernel(
@@ -956,11 +1040,13 @@ hipError_t gemm_w4a8_narrow(const int8_t* q, const float* xs, const uint8_t* cod
                             const uint8_t* group_scale, const float* codebook, const float* ws,
                             const void* bias, void* out, bool out_half, int M, int N, int K,
                             int config, hipStream_t s) {
-    // 1..2 rows by shape: the GEMV form; 3..16 (and 17..32 by the rule above) the row-tile
-    // kernel (the same bits as every tile config). The GEMV form's MFMA chains grow with the rows, the row tile's do not (graph
-    // replays over weights past the MALL, us GEMV / row tile: K=3072 N=12288 M=2 10.2 / 10.0,
-    // M=3 13.7 / 10.1, M=4 15.7 / 10.3; K=4096 N=14336 M=1 11.2 / 13.3, M=2 12.7 / 13.2, M=3
-    // 16.6 / 13.6; K=3072 N=3072 M=3 7.4 / 5.9).
+    // 1..2 rows by shape: the GEMV form; up to 64 the row-tile kernel (the same bits as every tile
+    // config). The GEMV form's MFMA chains grow with the rows, the row tile's do not (graph replays
+    // over weights past the MALL, us GEMV / row tile: K=3072 N=12288 M=2 10.2 / 10.0, M=3 13.7 /
+    // 9.1; K=4096 N=14336 M=1 11.2 / 13.3, M=2 12.7 / 13.2). Against the narrow tiles, whose N/64
+    // workgroups leave the chip idle and run K as one chain (us narrow / row tile): K=12288 N=3072
+    // M=2 64.0 / 11.3, M=16 64.1 / 14.7, M=64 63.6 / 30.9; K=3072 N=12288 M=64 21.7 / 18.3; K=3072
+    // N=3072 M=48 18.5 / 8.5; but K=256 N=14336 M=33 5.5 / 6.5.
     if (config < 0 && M <= kW4GemvRows && K <= kW4MaxK) {
         const W4 w4{group_scale, codebook};
         if (out_half)
@@ -969,14 +1055,14 @@ hipError_t gemm_w4a8_narrow(const int8_t* q, const float* xs, const uint8_t* cod
         return bias ? launch_w4a8_decode<false, true>(q, xs, codes, w4, ws, bias, out, M, N, K, s)
                     : launch_w4a8_decode<false, false>(q, xs, codes, w4, ws, bias, out, M, N, K, s);
     }
-    const bool two = M <= kW4Rows2Max && K <= kW4Rows2MaxK && static_cast<int64_t>(M) * K <= kW4Rows2Area;
-    if (config < 0 && ((M <= kW4RowsMax && K <= kW4MaxK) || two)) {
+    if (config < 0 && M <= kW4RowsMax && (M <= 32 || K >= kW4RowsK)) {
         const W4 w4{group_scale, codebook};
-        if (out_half)
-            return bias ? launch_w4a8_rows<true, true>(q, xs, codes, w4, ws, bias, out, M, N, K, s)
-                        : launch_w4a8_rows<true, false>(q, xs, codes, w4, ws, bias, out, M, N, K, s);
-        return bias ? launch_w4a8_rows<false, true>(q, xs, codes, w4, ws, bias, out, M, N, K, s)
-                    : launch_w4a8_rows<false, false>(q, xs, codes, w4, ws, bias, out, M, N, K, s);
+        switch ((M + 15) / 16) {
+            case 1: return launch_w4a8_rows<1>(q, xs, codes, w4, ws, bias, out, out_half, M, N, K, s);
+            case 2: return launch_w4a8_rows<2>(q, xs, codes, w4, ws, bias, out, out_half, M, N, K, s);
+            case 3: return launch_w4a8_rows<3>(q, xs, codes, w4, ws, bias, out, out_half, M, N, K, s);
+            default: return launch_w4a8_rows<4>(q, xs, codes, w4, ws, bias, out, out_half, M, N, K, s);
+        }
     }
     return narrow<true, true>(reinterpret_cast<const uint8_t*>(q), xs, codes, ws, bias, out, N,
                               out_half, M, N, K, 0, config < 0 ? narrow_config(M, N) : config, s,

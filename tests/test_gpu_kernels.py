@@ -905,8 +905,7 @@ def test_w4a8_unpack_every_scale_byte_bit_exact(ops, codebook):
                          ids=lambda s: "x".join(map(str, s)))  # fmt: skip
 def test_w4a8_linear_bit_exact(ops, shape, codebook):
     """The w4a8 linear (int8.convrot's operand; the GEMV form at 1..2 rows, the row-tile kernel
-    at 3..16 and, in two activation blocks, at 17..32 rows with M·K ≤ 98304 and K ≤ 4096, the
-    fused unpack-in-registers GEMM up to 256 rows, unpack + the int8 GEMM beyond)
+    to 64, the fused unpack-in-registers GEMM to 256 rows, unpack + the int8 GEMM beyond)
     equals the int8 CPU law on the unpacked levels, bit for bit, with and without bias; the
     fused and unpack configs agree bit for bit."""
     from cozyq import prebuilt
@@ -923,6 +922,33 @@ def test_w4a8_linear_bit_exact(ops, shape, codebook):
     unpacked = ops.w4a8_gemm(q, s, w, b.to(DEV), torch.bfloat16, prebuilt.UNPACK)
     for config in range(1, prebuilt.GEMM_CONFIGS):  # every fused tile
         assert torch.equal(ops.w4a8_gemm(q, s, w, b.to(DEV), torch.bfloat16, config), unpacked), config
+
+
+@pytest.mark.parametrize("shape", [(2, 136, 12288), (3, 1032, 14336), (16, 264, 12288), (17, 136, 8192),
+                                   (33, 136, 4096), (48, 8, 1024), (64, 1032, 12288), (65, 136, 1024),
+                                   (20, 4104, 2048), (48, 8200, 1024), (9, 12296, 1024), (64, 14336, 1280),
+                                   (5, 12296, 1280), (8, 9216, 512), (33, 264, 768), (7, 520, 32768)],
+                         ids=lambda s: "x".join(map(str, s)))  # fmt: skip
+def test_w4a8_row_tiles_bit_exact(ops, shape):
+    """The row-tile kernel at the edges of its dispatch: one to four weight tiles a workgroup (256
+    tiles and one more, 512, 768), one to four activation blocks, K in one pass and several with a
+    ragged last one, a last tile of 8 rows, in bf16 and fp16; bit for bit the unpack + int8 GEMM
+    path, and the CPU law on its first rows."""
+    from cozyq import prebuilt
+
+    m, n, k = shape
+    w, levels, scale = _w4a8(n, k, 77 + m, True)
+    gen = torch.Generator().manual_seed(m + n)
+    x = torch.randn(m, k, generator=gen).to(torch.bfloat16)
+    b = torch.randn(n, generator=gen).to(torch.bfloat16)
+    q, s = ops.int8_quantize(x.to(DEV))
+    for dtype in (torch.bfloat16, torch.float16):
+        for bias in (None, b.to(dtype).to(DEV)):
+            got = ops.w4a8_gemm(q, s, w, bias, dtype)
+            assert torch.equal(got, ops.w4a8_gemm(q, s, w, bias, dtype, prebuilt.UNPACK))
+    rows = min(m, 2)
+    got = ops.w4a8_gemm(q, s, w, b.to(DEV), torch.bfloat16)[:rows].cpu()
+    assert torch.equal(got, laws.int8_linear(x, levels, scale, b, torch.bfloat16)[:rows])
 
 
 # ------------------------------------------------------------------------ MXFP8 lane
