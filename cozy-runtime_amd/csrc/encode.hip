@@ -93,7 +93,7 @@ __global__ __launch_bounds__(kEncThreads) void encode_rotated_kernel(const void*
             *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
             *reinterpret_cast<float4*>(dst + 4) = make_float4(v[4], v[5], v[6], v[7]);
         }
-        rotate_lds_chunk<256, kEncThreads>(lds, width, tid, out, amax);
+        rotate_lds_chunk<256>(lds, width, tid, kEncThreads, out, amax);
         __syncthreads();
         return width / 256;
     };

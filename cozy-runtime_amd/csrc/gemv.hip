@@ -565,7 +565,7 @@ __global__ __launch_bounds__(kDThreads) void int8_decode_kernel(
                 *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
                 *reinterpret_cast<float4*>(dst + 4) = make_float4(v[4], v[5], v[6], v[7]);
             }
-            rotate_lds_chunk<256, kDThreads>(work, width, tid, rot[m][c4], amax[m]);
+            rotate_lds_chunk<256>(work, width, tid, kDThreads, rot[m][c4], amax[m]);
             __syncthreads();
         }
         amax[m] = wave_max(amax[m]);

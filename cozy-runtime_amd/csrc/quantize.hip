@@ -40,8 +40,21 @@ __device__ __forceinline__ void load8(const uint16_t* p, float* v) {
     }
 }
 
+// The sum over a wave, uniform, by DPP within 16-lane rows (wave_max's pattern), then the rows.
+__device__ __forceinline__ float wave_sum(float v) {
+    v += dpp_move<0xB1>(v);
+    v += dpp_move<0x4E>(v);
+    v += dpp_move<0x124>(v);
+    v += dpp_move<0x128>(v);
+    const int b = __builtin_bit_cast(int, v);
+    float r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 16 * i));
+    return (r[0] + r[1]) + (r[2] + r[3]);
+}
+
 __device__ __forceinline__ float block_sum(float v, float* red) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    v = wave_sum(v);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (lane == 0) red[wave] = v;
     __syncthreads();
@@ -66,34 +79,13 @@ __device__ __forceinline__ bool halves(const Prologue& p) {
     return p.act == kActSitu || (p.act == kActSwiglu && p.up == nullptr);
 }
 
-// Elements e..e+7 of row `row` after the prologue; `mean` and `rstd` are the row's norm
-// statistics (mean 0 for the RMS norm).
+// Elements e..e+7 of a row that is not [hidden | gate], already loaded into v, after the prologue.
 template <bool kHalf>
-__device__ __forceinline__ void load8_prologue(const Prologue& p, const uint16_t* x, int row,
-                                               int K, int e, float mean, float rstd, float* v) {
-    if (halves(p)) {
-        const uint16_t* xr = x + static_cast<int64_t>(row) * (2 * K);
-        float h[8], g[8];
-        load8<kHalf>(xr + e, h);
-        load8<kHalf>(xr + K + e, g);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            if (p.act == kActSitu) {
-                // rotate.cu:252: (4 tanh(g/4) / (1 + e^-g)) · (25 tanh(h/25))
-                v[i] = (4.0f * tanhf(g[i] * 0.25f) / (1.0f + expf(-g[i]))) * (25.0f * tanhf(h[i] / 25.0f));
-            } else {
-                // rotate.cu:271-282: silu(gate) in the row dtype (IEEE divide), times up, rounded again
-                const float silu = in_dtype<kHalf>(g[i] / (1.0f + expf(-g[i])));
-                v[i] = in_dtype<kHalf>(silu * h[i]);
-            }
-        }
-        return;
-    }
-    const int64_t at = static_cast<int64_t>(row) * K + e;
-    load8<kHalf>(x + at, v);
+__device__ __forceinline__ void finish8_prologue(const Prologue& p, int row, int K, int e, float mean,
+                                                 float rstd, float* v) {
     if (p.act == kActSwiglu) {  // gate rows in x, up rows in `up` (rotate.cu:260-268)
         float u[8];
-        load8<kHalf>(p.up + at, u);
+        load8<kHalf>(p.up + static_cast<int64_t>(row) * K + e, u);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const float silu = in_dtype<kHalf>(v[i] / (1.0f + expf(-v[i])));
@@ -130,6 +122,33 @@ __device__ __forceinline__ void load8_prologue(const Prologue& p, const uint16_t
     }
 }
 
+// Elements e..e+7 of row `row` after the prologue; `mean` and `rstd` are the row's norm
+// statistics (mean 0 for the RMS norm).
+template <bool kHalf>
+__device__ __forceinline__ void load8_prologue(const Prologue& p, const uint16_t* x, int row,
+                                               int K, int e, float mean, float rstd, float* v) {
+    if (halves(p)) {
+        const uint16_t* xr = x + static_cast<int64_t>(row) * (2 * K);
+        float h[8], g[8];
+        load8<kHalf>(xr + e, h);
+        load8<kHalf>(xr + K + e, g);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if (p.act == kActSitu) {
+                // rotate.cu:252: (4 tanh(g/4) / (1 + e^-g)) · (25 tanh(h/25))
+                v[i] = (4.0f * tanhf(g[i] * 0.25f) / (1.0f + expf(-g[i]))) * (25.0f * tanhf(h[i] / 25.0f));
+            } else {
+                // rotate.cu:271-282: silu(gate) in the row dtype (IEEE divide), times up, rounded again
+                const float silu = in_dtype<kHalf>(g[i] / (1.0f + expf(-g[i])));
+                v[i] = in_dtype<kHalf>(silu * h[i]);
+            }
+        }
+        return;
+    }
+    load8<kHalf>(x + static_cast<int64_t>(row) * K + e, v);
+    finish8_prologue<kHalf>(p, row, K, e, mean, rstd, v);
+}
+
 // The row's norm statistics (rotate.cu:204-221): the mean (layer norm; 0 for RMS) and
 // rsqrt(Σ(x - mean)² / K + eps) over x's K elements, every thread of the block taking part.
 template <bool kHalf>
@@ -163,8 +182,8 @@ __device__ __forceinline__ float2 norm_stats(const Prologue& p, const uint16_t* 
 }
 
 
-// Rotation by H_kRot (256: H4^⊗4 then ·1/16; 128: H2⊗H4^⊗3 unnormalized) and per-row int8.
-// One block per row; kMaxChunks bounds the row's 4096-element chunks held in registers.
+// Rotation by H_kRot (256: H4^⊗4 then ·1/16; 128: H2⊗H4^⊗3 unnormalized) and per-row int8 of
+// long rows. One block per row; kMaxChunks bounds the row's 4096-element chunks held in registers.
 template <bool kHalf, int kRot, int kMaxChunks, bool kPro = false>
 __global__ __launch_bounds__(kThreads) void rotate_quantize_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ q, float* __restrict__ scales, int K,
@@ -222,7 +241,7 @@ __global__ __launch_bounds__(kThreads) void rotate_quantize_kernel(
             *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
             *reinterpret_cast<float4*>(dst + 4) = make_float4(v[4], v[5], v[6], v[7]);
         }
-        rotate_lds_chunk<kRot, kThreads>(lds, width, tid, out[c], amax);
+        rotate_lds_chunk<kRot>(lds, width, tid, kThreads, out[c], amax);
         __syncthreads();
     }
     amax = block_max(amax, red);
@@ -238,25 +257,96 @@ __global__ __launch_bounds__(kThreads) void rotate_quantize_kernel(
             const int groups = min(kChunk, K - base) / kRot;
             const int g = tid / L::kRuns, hi = tid % L::kRuns;
             if (g >= groups) continue;
-            uint32_t packed[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                uint32_t word = 0;
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    word |= static_cast<uint32_t>(static_cast<uint8_t>(
-                                q8<decltype(fast)::value>(out[c][4 * i + j], scale, rs))) << (8 * j);
-                packed[i] = word;
-            }
+            constexpr bool kFast = decltype(fast)::value;
             *reinterpret_cast<uint4*>(qr + base + g * kRot + hi * 16) =
-                make_uint4(packed[0], packed[1], packed[2], packed[3]);
+                make_uint4(q8x4<kFast>(out[c], scale, rs), q8x4<kFast>(out[c] + 4, scale, rs),
+                           q8x4<kFast>(out[c] + 8, scale, rs), q8x4<kFast>(out[c] + 12, scale, rs));
         }
     };
     if (scale < __builtin_huge_valf()) emit(std::true_type{}); else emit(std::false_type{});
 }
 
-// Rows of at most kRowMaxK elements with no prologue: one wave per row (rows.h), no workgroup
-// barrier, and each wave's next row loaded while it rotates and quantizes the current one, so a
+// Rotation and per-row int8 of rows of at most 16·kBlockMax elements, one workgroup a row of as
+// many waves as the row fills, 16 contiguous elements a thread: the row is read once, held in registers through the prologue's
+// norm, and rotated in one pass through LDS. Bound: VALU at many rows (~18 instructions an element,
+// 11 of them the rotation's adds), the chain of one row's phases at few. Measured against a wave a
+// row with its next row's loads in flight (us, graph replays): K=3072 M=16 5.3 -> 3.2, M=1024 5.8
+// -> 4.6, M=4096 12.9 -> 10.5 (3.6 TB/s); K=1024 M=4096 6.6 -> 5.3; against 4096-element chunks one
+// after another: K=12288 M=16 5.9 -> 4.3; K=5120 M=4000 17.8 -> 15.2.
+constexpr int kBlockMax = 1024;
+
+template <bool kHalf, int kRot, bool kPro>
+__global__ __launch_bounds__(kBlockMax) void row_block_kernel(
+    const uint16_t* __restrict__ x, int8_t* __restrict__ q, float* __restrict__ scales, int K, Prologue pro) {
+    using L = Layout<kRot>;
+    extern __shared__ __attribute__((aligned(16))) float block_lds[];  // K / kRot groups
+    float* const lds = block_lds;
+    __shared__ float red[kBlockMax / 64];
+    const int row = blockIdx.x, tid = threadIdx.x, e = 16 * tid;
+    const bool live = e < K;
+    float v[16];
+    bool loaded = true;
+    if constexpr (kPro) loaded = !halves(pro);
+    if (loaded) {
+        const __amdgpu_buffer_rsrc_t xr = row_view(x + static_cast<int64_t>(row) * K, K);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)  // zeros past the row
+            unpack8<kHalf>(__builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(xr, 2 * e + 16 * h, 0, 0)), v + 8 * h);
+    }
+    if constexpr (kPro) {
+        if (!loaded) {
+            if (live) {
+                load8_prologue<kHalf>(pro, x, row, K, e, 0.0f, 1.0f, v);
+                load8_prologue<kHalf>(pro, x, row, K, e + 8, 0.0f, 1.0f, v + 8);
+            }
+        } else {
+            // rotate.cu:204-221: the mean (layer norm; 0 for RMS) and rsqrt(Σ(x - mean)² / K + eps).
+            float mean = 0.0f, rstd = 1.0f;
+            if (pro.norm == kNormLayer) {
+                float sum = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) sum += v[i];
+                mean = block_sum(sum, red) / static_cast<float>(K);
+            }
+            if (pro.norm != 0) {
+                float squares = 0.0f;
+                if (live) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        const float d = v[i] - mean;
+                        squares += d * d;
+                    }
+                }
+                rstd = rsqrtf(block_sum(squares, red) / static_cast<float>(K) + pro.eps);
+            }
+            if (live) {
+                finish8_prologue<kHalf>(pro, row, K, e, mean, rstd, v);
+                finish8_prologue<kHalf>(pro, row, K, e + 8, mean, rstd, v + 8);
+            }
+        }
+    }
+    if (live) {
+        float* dst = lds + L::at(tid / L::kRuns, tid % L::kRuns, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<float4*>(dst + 4 * i) = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+    }
+    float amax = 0.0f;
+    rotate_lds_chunk<kRot>(lds, K, tid, blockDim.x, v, amax);
+    amax = block_max(amax, red);
+    const float scale = fmaxf(amax / 127.0f, kScaleFloor);
+    if (tid == 0) scales[row] = kRot == 128 ? scale * 0.08838834764831845f : scale;
+    if (!live) return;
+    const float rs = 1.0f / scale;
+    uint4* dst = reinterpret_cast<uint4*>(q + static_cast<int64_t>(row) * K + e);
+    if (scale < __builtin_huge_valf())
+        *dst = make_uint4(q8x4<true>(v, scale, rs), q8x4<true>(v + 4, scale, rs), q8x4<true>(v + 8, scale, rs), q8x4<true>(v + 12, scale, rs));
+    else
+        *dst = make_uint4(q8x4<false>(v, scale, rs), q8x4<false>(v + 4, scale, rs), q8x4<false>(v + 8, scale, rs), q8x4<false>(v + 12, scale, rs));
+}
+
+// Unrotated rows of at most kRowMaxK elements with no prologue: one wave per row (rows.h), no
+// workgroup barrier, and each wave's next row loaded while it rotates and quantizes the current one, so a
 // CU keeps ~12 rows (72 KB at K = 3072) of loads in flight.
 constexpr int kRowWaves = 4;
 
@@ -329,9 +419,8 @@ __global__ __launch_bounds__(kThreads) void rowwise_quantize_kernel(
                 word[0] = e4m3x4(r[0], r[1], r[2], r[3]);
                 word[1] = e4m3x4(r[4], r[5], r[6], r[7]);
             } else {
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    word[i / 4] |= static_cast<uint32_t>(static_cast<uint8_t>(q8<kFast>(v[i], scale, rs))) << (8 * (i % 4));
+                word[0] = q8x4<kFast>(v, scale, rs);
+                word[1] = q8x4<kFast>(v + 4, scale, rs);
             }
             *reinterpret_cast<uint2*>(qr + e) = make_uint2(word[0], word[1]);
         }
@@ -409,17 +498,16 @@ __global__ __launch_bounds__(kThreads) void mx_quantize_kernel(
 template <bool kHalf, int kRot, bool kPro>
 hipError_t launch_rotated(const void* x, int8_t* q, float* scales, int M, int K,
                           const Prologue& pro, hipStream_t s) {
-    const int chunks = (K + kChunk - 1) / kChunk;
-    const dim3 grid(M), block(kThreads);
+    const dim3 grid(M);
     auto xp = static_cast<const uint16_t*>(x);
-    if (chunks <= 1)
-        rotate_quantize_kernel<kHalf, kRot, 1, kPro><<<grid, block, 0, s>>>(xp, q, scales, K, pro);
-    else if (chunks <= 2)
-        rotate_quantize_kernel<kHalf, kRot, 2, kPro><<<grid, block, 0, s>>>(xp, q, scales, K, pro);
-    else if (chunks <= 4)
-        rotate_quantize_kernel<kHalf, kRot, 4, kPro><<<grid, block, 0, s>>>(xp, q, scales, K, pro);
+    // 9..16 waves a row synchronize too often for many rows: there the 4-wave chunked form streams
+    // better (K=12288 M=4096 38.0 us against 34.7; M=512 7.5 against 9.1).
+    if (!kPro && K > 8192 && K <= 4 * kChunk && M > 1024)
+        rotate_quantize_kernel<kHalf, kRot, 4, kPro><<<grid, kThreads, 0, s>>>(xp, q, scales, K, pro);
+    else if (K <= 16 * kBlockMax)
+        row_block_kernel<kHalf, kRot, kPro><<<grid, 64 * ((K + 1023) / 1024), K / kRot * Layout<kRot>::kGroupStride * 4, s>>>(xp, q, scales, K, pro);
     else
-        rotate_quantize_kernel<kHalf, kRot, 8, kPro><<<grid, block, 0, s>>>(xp, q, scales, K, pro);
+        rotate_quantize_kernel<kHalf, kRot, 8, kPro><<<grid, kThreads, 0, s>>>(xp, q, scales, K, pro);
     return hipGetLastError();
 }
 
@@ -451,15 +539,12 @@ hipError_t rotate_quantize(const void* x, bool x_half, int8_t* q, float* scales,
                       : launch_rotated<false, 256, true>(x, q, scales, M, K, *pro, s);
     }
     const Prologue none{};
-    if (K <= kRowMaxK && (rotation == 0 || rotation == 128 || rotation == 256)) {
+    if (K <= kRowMaxK && rotation == 0) {
         // 12 waves a CU: three 4-wave blocks on each of the 256 CUs, grid-strided over the rows.
         const int blocks = min((M + kRowWaves - 1) / kRowWaves, 3 * 256);
         auto xp = static_cast<const uint16_t*>(x);
-#define COZYQ_ROWS(H, R) row_quantize_kernel<H, R><<<blocks, 64 * kRowWaves, 0, s>>>(xp, q, scales, M, K)
-        if (rotation == 0) { if (x_half) COZYQ_ROWS(true, 0); else COZYQ_ROWS(false, 0); }
-        else if (rotation == 128) { if (x_half) COZYQ_ROWS(true, 128); else COZYQ_ROWS(false, 128); }
-        else { if (x_half) COZYQ_ROWS(true, 256); else COZYQ_ROWS(false, 256); }
-#undef COZYQ_ROWS
+        if (x_half) row_quantize_kernel<true, 0><<<blocks, 64 * kRowWaves, 0, s>>>(xp, q, scales, M, K);
+        else row_quantize_kernel<false, 0><<<blocks, 64 * kRowWaves, 0, s>>>(xp, q, scales, M, K);
         return hipGetLastError();
     }
     if (rotation == 0) {

@@ -37,16 +37,16 @@ __device__ __forceinline__ void h4(float& a, float& b, float& c, float& d) {
 // into `lds` (Layout<kRot>): a barrier, the outer two stages (thread = one column of a group's
 // runs), a barrier, then the inner two stages on the thread's contiguous 16-run (group
 // tid / runs, run tid % runs) into `w`, scaled by 1/16 for kRot = 256, and its |max| into
-// `amax`. Threads past the chunk's groups leave `w` untouched. The caller barriers before
+// `amax`. `threads` take part; those past the chunk's groups leave `w` untouched. The caller barriers before
 // writing `lds` again.
-template <int kRot, int kThreads>
-__device__ __forceinline__ void rotate_lds_chunk(float* lds, int width, int tid, float (&w)[16],
+template <int kRot>
+__device__ __forceinline__ void rotate_lds_chunk(float* lds, int width, int tid, int threads, float (&w)[16],
                                                  float& amax) {
     using L = Layout<kRot>;
     __syncthreads();
     // Phase 2: the outer two stages; thread holds one column `t` of a group's runs.
     const int groups = width / kRot;
-    for (int task = tid; task < groups * 16; task += kThreads) {
+    for (int task = tid; task < groups * 16; task += threads) {
         const int g = task / 16, t = task % 16;
         float v[L::kRuns];
 #pragma unroll
@@ -99,6 +99,30 @@ __device__ __forceinline__ int8_t q8(float v, float scale, float rs) {
     float r = __builtin_rintf(kFast ? div_rn(v, scale, rs) : v / scale);
     r = fminf(fmaxf(r, -127.0f), 127.0f);
     return static_cast<int8_t>(static_cast<int>(r));
+}
+
+// Four codes of q8 packed little-endian. The fast form leaves out what a code cannot show (the
+// sign of a zero quotient) and rounds by adding 1.5·2^23, which leaves the integer, half to even,
+// in the sum's low byte: 6 VALU instructions a code where 9 ran, and the quantizers are VALU-bound
+// at many rows. A NaN gives -127, as the clamp of q8 does.
+template <bool kFast>
+__device__ __forceinline__ uint32_t q8x4(const float* v, float scale, float rs) {
+    if constexpr (kFast) {
+        uint32_t m[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float q = v[j] * rs;
+            const float r = __builtin_fmaf(__builtin_fmaf(-q, scale, v[j]), rs, q);  // div_rn
+            m[j] = bits_of(__builtin_amdgcn_fmed3f(r, -127.0f, 127.0f) + 12582912.0f);
+        }
+        return __builtin_amdgcn_perm(m[1], m[0], 0x0c0c0400u) | __builtin_amdgcn_perm(m[3], m[2], 0x04000c0cu);
+    } else {
+        uint32_t word = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            word |= static_cast<uint32_t>(static_cast<uint8_t>(q8<false>(v[j], scale, rs))) << (8 * j);
+        return word;
+    }
 }
 
 }  // namespace cozyq

@@ -67,16 +67,6 @@ __device__ __forceinline__ void unpack8(const uint4& raw, float* v) {
     }
 }
 
-// Four codes of q8 packed little-endian.
-template <bool kFast>
-__device__ __forceinline__ uint32_t q8x4(const float* v, float scale, float rs) {
-    uint32_t word = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-        word |= static_cast<uint32_t>(static_cast<uint8_t>(q8<kFast>(v[j], scale, rs))) << (8 * j);
-    return word;
-}
-
 // One row (K <= kRowMaxK, K % max(kRot, 16) == 0) held in `raw` by row_loads, rotated by H_kRot
 // (256: H4^⊗4 then ·1/16; 128: H2⊗H4^⊗3 unnormalized, 1/√128 folded into the scale; 0: none),
 // quantized per row into `qr` and its scale into `*scale_out` (lane 0). `lds` is the wave's
@@ -183,16 +173,20 @@ __device__ __forceinline__ void quantize_row_wave(const uint4 (&raw)[kRowLoads],
                     for (int d3 = 0; d3 < 4; ++d3) h4(o[4 * d3], o[4 * d3 + 1], o[4 * d3 + 2], o[4 * d3 + 3]);
 #pragma unroll
                     for (int i = 0; i < 16; ++i) {
-                        if constexpr (kRot == 256) o[i] = o[i] * 0.0625f;  // .mul_(1.0 / 16), exact
                         amax = fmaxf(amax, fabsf(o[i]));
                     }
                 }
             }
             wave_lds_sync();  // the next pass (or row) writes the slice again
         }
-        amax = wave_max(amax);
-        const float scale = fmaxf(amax / 127.0f, kScaleFloor);
-        if (lane == 0) *scale_out = kRot == 128 ? scale * 0.08838834764831845f : scale;
+        // The law's .mul_(1.0 / 16) of the 256 rotation scales row and maximum alike by a power of
+        // two: the codes come from the unscaled row over 16 times the scale (the same quotients;
+        // where the multiply would underflow the quotient rounds to 0 either way).
+        constexpr float kUnit = kRot == 256 ? 16.0f : 1.0f;
+        amax = wave_max(amax) * (1.0f / kUnit);
+        const float row_scale = fmaxf(amax / 127.0f, kScaleFloor);
+        if (lane == 0) *scale_out = kRot == 128 ? row_scale * 0.08838834764831845f : row_scale;
+        const float scale = kUnit * row_scale;
         const float rs = 1.0f / scale;
         auto emit = [&](auto fast) {
             constexpr bool kFast = decltype(fast)::value;

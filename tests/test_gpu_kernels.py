@@ -391,6 +391,28 @@ def test_int8_quantize_bit_exact(ops, rotation, dtype, shape):
     assert torch.equal(s.cpu().view(torch.int32), ws.reshape(-1).view(torch.int32))
 
 
+@pytest.mark.parametrize("rotation", [256, 128])
+@pytest.mark.parametrize("shape", [(1, 1024), (2, 1280), (7, 8192), (9, 8448), (1025, 8448), (1025, 12288), (5, 16384),
+                                   (1030, 16384), (3, 16640), (1024, 12288)],
+                         ids=lambda s: f"{s[0]}x{s[1]}")  # fmt: skip
+def test_int8_row_block_edges_bit_exact(ops, rotation, shape):
+    """The rotated quantizer at the edges of its dispatch (a workgroup of 1, 2, 8, 9 and 16 waves a
+    row; 4096-element chunks past 8192 with more than 1024 rows and past 16384 always), with rows
+    that hold an infinity, only zeros, and subnormal-scale values: the law's codes and scales."""
+    m, k = shape
+    x = activations(m, k, seed=k + m)
+    x[0, 3] = 0.0 if m == 1 else float("inf")
+    if m > 2:
+        x[1] = 0.0
+        x[2] = (x[2].float() * 1e-38).to(x.dtype)
+    q, s = ops.int8_quantize_rot(x.to(DEV), rotation)
+    wq, ws = laws.quantize_rows_int8(x, rotation)
+    finite = torch.isfinite(ws.reshape(-1))
+    assert torch.equal(s.cpu().view(torch.int32)[finite], ws.reshape(-1).view(torch.int32)[finite])
+    assert torch.equal(q.cpu()[finite], wq[finite])
+    assert torch.equal(torch.isfinite(s.cpu()), finite)
+
+
 @pytest.mark.parametrize("rotation", [256, 128, 0])
 @pytest.mark.parametrize("shape", [(4100, 2304), (3073, 4096), (6500, 768), (2, 1280)],
                          ids=lambda s: f"{s[0]}x{s[1]}")
