@@ -111,12 +111,15 @@ class _QuantizedLane(_Lane):
     def quantize(self, torch: Any, x: Tensor) -> PreQuantized | None:
         return int8_linear.quantize(torch, x)
 
+    # (The buffers by name: a module's attribute miss costs more than reading all three.)
     def gemm(self, torch, leaf, operand, out_dtype, out):
-        return int8_linear.gemm(torch, operand, read(leaf.data), read(leaf.scale), read(leaf.bias),
+        held = leaf._buffers
+        return int8_linear.gemm(torch, operand, read(held["data"]), read(held["scale"]), read(held["bias"]),
                                 out_dtype, out)  # fmt: skip
 
     def linear(self, torch, leaf, x, out_dtype):
-        return int8_linear.linear(torch, x, read(leaf.data), read(leaf.scale), read(leaf.bias), out_dtype)
+        held = leaf._buffers
+        return int8_linear.linear(torch, x, read(held["data"]), read(held["scale"]), read(held["bias"]), out_dtype)
 
     def run(self, torch, leaf, x, prequantized, out):
         if isinstance(x, PreQuantized):
@@ -141,11 +144,13 @@ class _Fp8Lane(_QuantizedLane):
         return fp8_linear.quantize(torch, x)
 
     def gemm(self, torch, leaf, operand, out_dtype, out):
-        return fp8_linear.gemm(torch, operand, read(leaf.data), read(leaf.scale), read(leaf.bias),
+        held = leaf._buffers
+        return fp8_linear.gemm(torch, operand, read(held["data"]), read(held["scale"]), read(held["bias"]),
                                out_dtype, out)  # fmt: skip
 
     def linear(self, torch, leaf, x, out_dtype):
-        return fp8_linear.linear(torch, x, read(leaf.data), read(leaf.scale), read(leaf.bias), out_dtype)
+        held = leaf._buffers
+        return fp8_linear.linear(torch, x, read(held["data"]), read(held["scale"]), read(held["bias"]), out_dtype)
 
 
 class _W4a8Lane(_QuantizedLane):

@@ -108,7 +108,7 @@ class W4a8:
 
 
 def _ptr(t: Tensor | None) -> int | None:
-    return None if t is None else int(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _stride(t: Tensor | None) -> int:
@@ -118,8 +118,9 @@ def _stride(t: Tensor | None) -> int:
 def _aligned(t: Tensor) -> Tensor:
     """`t` contiguous at a 16-byte address: the epilogues read scales and biases 16 bytes at a
     time."""
-    t = t.contiguous()
-    return t if t.data_ptr() % 16 == 0 else t.clone()
+    if not t.is_contiguous():
+        t = t.contiguous()
+    return t.clone() if t.data_ptr() & 15 else t
 
 
 @dataclass(slots=True)
@@ -132,6 +133,13 @@ class Prebuilt:
     _lib: Any = field(init=False)
     #: 16-bit dtype -> whether it is fp16 (the kernels' `half` flag).
     _halves: dict[Any, bool] = field(init=False, default_factory=dict)
+    #: What a call reads of the library and of torch, looked up once: the codes it answers, its
+    #: limits, and the raw handle of a card's current stream.
+    _declined: int = field(init=False)
+    _out_of_memory: int = field(init=False)
+    _gemv_rows: int = field(init=False)
+    _widest: int = field(init=False)
+    _current_stream: Any = field(init=False)
     #: The fused linear's counters, one zeroed int32 buffer per stream (each call leaves its
     #: buffer zero; calls on one stream run in order, so they share it).
     _workspaces: dict[int, Tensor] = field(init=False, default_factory=dict)
@@ -141,6 +149,11 @@ class Prebuilt:
     def __post_init__(self) -> None:
         self._lib = _lib.load()
         self._halves = {self.torch.bfloat16: False, self.torch.float16: True}
+        self._declined = int(self._lib.cozyq_not_supported())
+        self._out_of_memory = int(self._lib.cozyq_out_of_memory())
+        self._gemv_rows = int(self._lib.cozyq_gemv_rows())
+        self._widest = int(self._lib.cozyq_max_k())
+        self._current_stream = self.torch._C._cuda_getCurrentRawStream
 
     # ------------------------------------------------------------------ reference surface
 
@@ -167,7 +180,7 @@ class Prebuilt:
         (`cozyq_gemv`), or None where it declines (more rows, rows too wide for it, or a shape
         where quantize + GEMM is faster, `gemv_serves`)."""
         rows, width = flat.shape
-        if rows > self._lib.cozyq_gemv_rows() or not gemv_serves(rows, width):
+        if rows > self._gemv_rows or not gemv_serves(rows, width):
             return None
         out = self.torch.empty(shape, dtype=out_dtype, device=flat.device)
         if rows == 0:
@@ -177,7 +190,7 @@ class Prebuilt:
             _ptr(bias), out.data_ptr(), self._half(out_dtype), rows, data.shape[0], width,
             self._stream(),
         )  # fmt: skip
-        if code == self._lib.cozyq_not_supported():
+        if code == self._declined:
             return None
         self._check(code, "the GEMV")
         return out
@@ -205,7 +218,7 @@ class Prebuilt:
             scales.data_ptr(), data.data_ptr(), scale.data_ptr(), _ptr(bias), out.data_ptr(), n,
             self._half(out_dtype), rows, n, width, epilogue, work.data_ptr(), stream,
         )  # fmt: skip
-        if code == self._lib.cozyq_not_supported():
+        if code == self._declined:
             return None
         self._check(code, "the fused linear")
         return out, q, scales
@@ -254,7 +267,7 @@ class Prebuilt:
                 scale.data_ptr(), _ptr(bias), out.data_ptr(), self._half(out_dtype), rows,
                 data.shape[0], width, self._stream(),
             )  # fmt: skip
-            if code != self._lib.cozyq_not_supported():
+            if code != self._declined:
                 self._check(code, "the fp8 linear")
                 return out
         q, scales = self.fp8_quantize(flat)
@@ -305,7 +318,7 @@ class Prebuilt:
             w.group_scale.data_ptr(), _ptr(w.codebook), w.scale.data_ptr(), _ptr(bias),
             out.data_ptr(), self._half(out_dtype), rows, n, width, config, self._stream(),
         )  # fmt: skip
-        if code == self._lib.cozyq_not_supported() and config >= 0:
+        if code == self._declined and config >= 0:
             raise ValueError(f"w4a8_gemm: config {config} cannot take {rows}x{width}")
         self._check(code, "the w4a8 GEMM")
         return out
@@ -746,27 +759,23 @@ class Prebuilt:
         flat = self._rows(f, x, width)
         rows = flat.shape[0]
         plain = not norm and scale is None and shift is None
-        refusals = (
-            (gated and (x.shape[-1] % 2 or not plain),
-             f"{f.name}_quantize: a gated activation takes [hidden | gate] rows alone"),
-            (up is not None and (activation != SWIGLU or up.shape != x.shape or up.dtype != x.dtype or not plain),
-             f"{f.name}_quantize: SwiGLU takes gate and up rows of one shape alone"),
-        )  # fmt: skip
-        for refused, text in refusals:
-            if refused:
-                raise ValueError(text)
+        if gated and (x.shape[-1] % 2 or not plain):
+            raise ValueError(f"{f.name}_quantize: a gated activation takes [hidden | gate] rows alone")
+        if up is not None and (activation != SWIGLU or up.shape != x.shape or up.dtype != x.dtype or not plain):
+            raise ValueError(f"{f.name}_quantize: SwiGLU takes gate and up rows of one shape alone")
         other = None if up is None else self._rows(f, up)
         q = torch.empty(rows, width, dtype=torch.float8_e4m3fn if f.fp8 else torch.int8,
                         device=x.device)  # fmt: skip
         scales = torch.empty(rows, dtype=torch.float32, device=x.device)
-        tables = [self._table(t, flat) for t in (scale, shift)]
-        entries = next((t.shape[0] for t in tables if t is not None), rows) or 1
-        if any(t is not None and t.shape[0] != entries for t in tables) or rows % entries:
+        scale, shift = self._table(scale, flat), self._table(shift, flat)
+        first = shift if scale is None else scale
+        entries = (rows if first is None else first.shape[0]) or 1
+        if (shift is not None and shift.shape[0] != entries) or rows % entries:
             raise ValueError(f"{f.name}_quantize: modulation rows do not divide {rows} rows")
         code = self._lib.cozyq_quantize(
             self.index, f.fp8, flat.data_ptr(), self._half(flat.dtype), q.data_ptr(),
-            scales.data_ptr(), rows, width, _ptr(tables[0]), _ptr(tables[1]),
-            _stride(tables[0]), _stride(tables[1]), max(rows // entries, 1), norm, eps,
+            scales.data_ptr(), rows, width, _ptr(scale), _ptr(shift), _stride(scale),
+            _stride(shift), max(rows // entries, 1), norm, eps,
             activation, _ptr(other), self._stream(),
         )  # fmt: skip
         self._check(code, "the quantization")
@@ -798,49 +807,53 @@ class Prebuilt:
         bias = self._weight(f, data, scale, bias, width, out_dtype)
         scale = _aligned(scale)
         n = data.shape[0]
-        direct = out is not None and Placement(rows, n, out_dtype, q.device).takes(out)
-        result = out if direct and out is not None else torch.empty(
-            rows, n, dtype=out_dtype, device=q.device)
+        if out is not None and Placement(rows, n, out_dtype, q.device).takes(out):
+            result, ldo = out, out.stride(0)
+        else:
+            result, ldo = torch.empty(rows, n, dtype=out_dtype, device=q.device), n
         if rows == 0:
             return _landed(result, out)
-        if epilogue == 0 and f in (INT8, FP8):
+        if epilogue == 0 and (f is INT8 or f is FP8):
             code = self._lib.cozyq_gemm(
                 self.index, FAMILIES.index(self.family), f.fp8, q.data_ptr(), scales.data_ptr(),
                 data.data_ptr(), scale.data_ptr(), _ptr(bias), result.data_ptr(),
-                result.stride(0), self._half(out_dtype), rows, n, width, config, None, None,
+                ldo, self._half(out_dtype), rows, n, width, config, None, None,
                 self._stream(),
             )  # fmt: skip
         else:
             code = self._lib.cozyq_gemm_ex(
                 self.index, f.fp8, q.data_ptr(), scales.data_ptr(), data.data_ptr(),
-                scale.data_ptr(), _ptr(bias), result.data_ptr(), result.stride(0),
+                scale.data_ptr(), _ptr(bias), result.data_ptr(), ldo,
                 self._half(out_dtype), rows, n, width, epilogue, self._stream(),
             )  # fmt: skip
-        if code == self._lib.cozyq_not_supported() and config >= 0:
+        if code == self._declined and config >= 0:
             raise ValueError(f"{f.name}_gemm: config {config} cannot take {rows}x{width}")
         self._check(code, "the GEMM")
         return _landed(result, out)
 
     def _operand(self, op: str, code: Dtype, q: Tensor, scales: Tensor) -> tuple[int, int]:
         """Contract V3: a quantized operand, codes `q` [M, K] and float32 row scales; (M, K)."""
-        admit((q, Operand(kinds=(code,), extents=(None, None), dense=True, align=16),
-               every(f"{op}: q must be a contiguous, aligned {code} [M, K]")))  # fmt: skip
-        rows, width = (int(d) for d in q.shape)
-        admit((scales, Operand(kinds=(self.torch.float32,), count=rows, dense=True),
-               every(f"{op}: scales must be contiguous float32 with {rows} values")))  # fmt: skip
+        # The properties are asked in line; `admit` names the broken one.
+        if q.dtype is not code or q.dim() != 2 or not q.is_contiguous() or q.data_ptr() & 15:
+            admit((q, Operand(kinds=(code,), extents=(None, None), dense=True, align=16),
+                   every(f"{op}: q must be a contiguous, aligned {code} [M, K]")))  # fmt: skip
+        rows, width = q.shape
+        if scales.dtype is not self.torch.float32 or scales.numel() != rows or not scales.is_contiguous():
+            admit((scales, Operand(kinds=(self.torch.float32,), count=rows, dense=True),
+                   every(f"{op}: scales must be contiguous float32 with {rows} values")))  # fmt: skip
         return rows, width
 
     def _rows(self, f: _Format, x: Tensor, width: int | None = None) -> Tensor:
         """Contract V1 (`internal/prebuilt.py:360-370`): x on this card, each row quantizing to
         `width` elements (x's last extent unless given) that the kernels take; the rows as one
         contiguous matrix at a 16-byte address."""
-        width = int(x.shape[-1] if width is None else width)
-        limit = int(self._lib.cozyq_max_k())
-        if off_card(self.index, x):
+        if width is None:
+            width = x.shape[-1]
+        if x.get_device() != self.index:
             raise ValueError(f"{f.name}: x must be on cuda:{self.index}")
-        if width > limit or width % f.multiple:
-            raise ValueError(f"{f.name}: K must be a multiple of {f.multiple} up to {limit}, not {width}")
-        return _aligned(x.reshape(-1, x.shape[-1]))
+        if width > self._widest or width % f.multiple:
+            raise ValueError(f"{f.name}: K must be a multiple of {f.multiple} up to {self._widest}, not {width}")
+        return _aligned(x if x.dim() == 2 else x.reshape(-1, x.shape[-1]))
 
     def _weight(
         self, f: _Format, data: Tensor, scale: Tensor, bias: Tensor | None, width: int,
@@ -850,19 +863,34 @@ class Prebuilt:
         float32 row scales) on this card, a 16-bit output dtype, and `bias` in it."""
         torch = self.torch
         code = torch.float8_e4m3fn if f.fp8 else torch.int8
+        # The properties are asked in line (a call of a microsecond's work asks a dozen); `admit`
+        # names the first that is broken.
+        if (data.dtype is not code or data.dim() != 2 or data.shape[1] != width or not data.is_contiguous()
+                or data.data_ptr() & 15 or data.shape[0] & 7 or scale.dtype is not torch.float32
+                or scale.numel() != data.shape[0] or not scale.is_contiguous()):  # fmt: skip
+            self._refuse_weight(f, code, data, scale, width)
+        n = data.shape[0]
+        index = self.index
+        if (data.get_device() != index or scale.get_device() != index
+                or (bias is not None and bias.get_device() != index)):  # fmt: skip
+            raise ValueError(f"{f.name}: the weight's tensors must be on cuda:{index}")
+        self._half(out_dtype)
+        if bias is None:
+            return None
+        if bias.numel() != n:
+            raise ValueError(f"{f.name}: bias must have {n} values")
+        return _aligned(bias if bias.dtype is out_dtype else bias.to(out_dtype))
+
+    def _refuse_weight(self, f: _Format, code: Dtype, data: Tensor, scale: Tensor, width: int) -> None:
+        """Contract V2's refusals: a ValueError naming the first property that `data` or `scale`
+        breaks."""
         admit((data, Operand(kinds=(code,), extents=(None, width), dense=True, align=16, rows=8),
                {**every(f"{f.name}: data must be {code} [N, {width}]", KIND, EXTENT),
                 **every(f"{f.name}: data must be contiguous, aligned, N a multiple of 8", LAYOUT, ALIGN, ROWS)}))
         n = int(data.shape[0])
-        admit((scale, Operand(kinds=(torch.float32,), count=n, dense=True),
+        admit((scale, Operand(kinds=(self.torch.float32,), count=n, dense=True),
                {**every(f"{f.name}: scale must be float32 with {n} values", KIND, EXTENT),
                 LAYOUT: f"{f.name}: scale must be contiguous"}))  # fmt: skip
-        if off_card(self.index, data, scale, bias):
-            raise ValueError(f"{f.name}: the weight's tensors must be on cuda:{self.index}")
-        self._half(out_dtype)
-        if bias is not None and bias.numel() != n:
-            raise ValueError(f"{f.name}: bias must have {n} values")
-        return None if bias is None else _aligned(bias.to(out_dtype))
 
     # -------------------------------------------------------------- LoRA bake
 
@@ -1036,14 +1064,14 @@ class Prebuilt:
 
     def _stream(self) -> int:
         """The raw handle of torch's current stream on this card, which every launch uses."""
-        return int(self.torch.cuda.current_stream(self.index).cuda_stream)
+        return self._current_stream(self.index)
 
     def _check(self, code: int, what: str) -> None:
         """`internal/prebuilt.py:428-434`."""
         if code == 0:
             return
         detail = f"8-bit linear: {what}: {_lib.error_name(code)}"
-        if code == self._lib.cozyq_out_of_memory():
+        if code == self._out_of_memory:
             raise self.torch.cuda.OutOfMemoryError(detail)
         raise RuntimeError(detail)
 
