@@ -89,8 +89,9 @@ typedef void* (*cozyq_allocate_fn)(size_t bytes, void* context);
  * 2 128x64, 3 64x64, 4 32x64, 5 256x192 (rows x columns); -1 chooses by shape
  * (cozyq_gemm_config; int8 at 1..4 rows with no epilogue activation takes a GEMV on the
  * quantized rows where K <= 32768 / 16384 / 12288 at 1 / 2 / 3..4 rows, and at 5..32 rows with
- * K <= 4096 and N <= 4096 a 16-row weight tile); 6 and above return
- * hipErrorNotSupported. Every config gives the same int8 output bit for bit.
+ * K <= 4096 and N <= 4096 a 16-row weight tile; and shapes whose grid fills neither the narrow
+ * tiles' nor the 256-row tiles' rounds a tile of 32..192 rows x 64..256 columns between them); 6
+ * and above return hipErrorNotSupported. Every config gives the same int8 output bit for bit.
  * N % 8 == 0; K % 256 (int8) or K % 16 (fp8). */
 int cozyq_gemm(int device, int family, int fp8, const void* q, const float* scales,
                const void* w, const float* w_scale, const void* bias, void* out, int64_t ldo,
@@ -98,7 +99,7 @@ int cozyq_gemm(int device, int family, int fp8, const void* q, const float* scal
                void* allocate_context, void* stream);
 
 /* The config cozyq_gemm (and cozyq_gemm_ex, which always chooses) runs for config -1 at this
- * shape (reference: the `choose` of gemm_sm80.cu:283-288 and gemm_fp8.cu:23-29, which the
+ * shape, where config -1 takes one of the table's tiles (reference: the `choose` of gemm_sm80.cu:283-288 and gemm_fp8.cu:23-29, which the
  * reference does not export); -1 for a non-positive dimension. */
 int cozyq_gemm_config(int fp8, int M, int N, int K);
 

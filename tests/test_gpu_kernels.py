@@ -689,6 +689,59 @@ def test_every_gemm_config_bit_equal(ops, shape, dtype):
         assert_close(outs[0], laws.fp8_exact(x, f8, f8s, b))
 
 
+#: Shapes the rule gives a mid-size tile, one a tile, with ragged M, N and K among them.
+MID_SHAPES = [(66, 10976, 256), (130, 11152, 256), (193, 10888, 272), (261, 11056, 144), (326, 10896, 256),
+              (385, 13120, 512), (513, 13208, 256), (648, 13128, 144), (200, 3072, 4224), (300, 3080, 5136)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("shape", MID_SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_mid_tiles_bit_equal(ops, shape, dtype):
+    """The shape rule's mid-size tiles: int8 equals the law's product bit for bit (bias, and a
+    strided `out`), fp8 the 256x256 config's bits, with and without bias and tanh-GELU."""
+    m, n, k = shape
+    x = activations(m, k, seed=m * 5 + k)
+    data, scale = laws.int8_weight_rowwise(weights(n, k, seed=n))
+    b = (torch.randn(n, generator=torch.Generator().manual_seed(n)) * 0.1).to(dtype)
+    q, s = ops.int8_quantize_rot(x.to(DEV), 0)
+    rows = sorted({0, 1, m // 2, m - 17, m - 1})
+    for bias in (None, b):
+        want = laws.int8_product(q.cpu()[rows], s.cpu()[rows], data, scale, dtype)
+        want = want if bias is None else want + bias
+        wide = torch.full((m, n + 64), 7.0, dtype=dtype, device=DEV)
+        dev = None if bias is None else bias.to(DEV)
+        got = ops.int8_gemm_ex(q, s, data.to(DEV), scale.to(DEV), dev, dtype, out=wide[:, :n])
+        assert torch.equal(got[rows].cpu(), want)
+        assert bool((wide[:, n:] == 7.0).all())
+    gelu = ops.int8_gemm_ex(q, s, data.to(DEV), scale.to(DEV), b.to(DEV), dtype, epilogue=1)
+    assert_close(gelu[rows], laws.gelu_tanh(want.float()).double())
+    f8, f8s = laws.fp8_weight(weights(n, k, seed=n + 1))
+    q8, s8 = ops.fp8_quantize(x.to(DEV))
+    for bias in (None, b.to(DEV)):
+        got = ops.fp8_gemm(q8, s8, f8.to(DEV), f8s.to(DEV), bias, dtype)
+        assert torch.equal(got, ops.fp8_gemm(q8, s8, f8.to(DEV), f8s.to(DEV), bias, dtype, 0))
+    assert_close(got[rows], laws.fp8_exact(x[rows], f8, f8s, b))
+
+
+@pytest.mark.parametrize("shape", [(1, 616, 128), (65, 8328, 128), (66, 11024, 384), (131, 11032, 640), (193, 10912, 896),
+                                   (259, 10928, 128), (323, 10920, 256), (386, 13176, 512), (521, 13168, 1152),
+                                   (806, 12344, 128), (40, 264, 8192), (300, 1032, 2176)],
+                         ids=lambda s: "x".join(map(str, s)))  # fmt: skip
+def test_mx_mid_tiles(ops, shape):
+    """The MX GEMM on the rule's mid-size tiles (one to sixty-four K steps, scale blocks of four
+    steps whole and ragged) against the float64 product of the law's codes, with and without bias."""
+    m, n, k = shape
+    x = activations(m, k, seed=m + k)
+    x[:, : k // 2] *= 300.0  # block scales far apart within a row
+    data, wscales = laws.mx_quantize(weights(n, k, seed=n))
+    q, qs = ops.mx_quantize(x.to(DEV))
+    rows = sorted({0, m // 3, max(m - 17, 0), m - 1})
+    b = torch.randn(n, generator=torch.Generator().manual_seed(n)).to(torch.bfloat16)
+    for bias in (None, b):
+        got = ops.mx_gemm(q, qs, data.to(DEV), wscales.to(DEV), None if bias is None else bias.to(DEV), torch.bfloat16)
+        assert_close(got[rows], laws.mx_exact(x[rows], data, wscales, bias))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 def test_partial_last_round_runs_half_width_tiles_bit_equal(ops, dtype):
     """Config 0 on a grid whose last round is at most half full (M=4096, N=4352: 272 tiles of
