@@ -184,130 +184,183 @@ __global__ __launch_bounds__(64 * kGemvWaves) void nvfp4_gemv_kernel(const uint1
     }
 }
 
-// The row-block form for 5..64 rows (K % 128 == 0): a workgroup of 4 waves takes 64 weight rows,
-// each wave 16 of them over all of K, so no partial sums meet; the activation's 16·kMB rows come
-// through LDS in 512-column chunks (LDS-DMA, a ring of 3 up to 32 rows, else 2), read once per
-// workgroup instead of once per wave, and a wave keeps kRowsAhead macro steps of its codes and
-// scales in flight in registers.
-// Per macro step a lane decodes its row's 32 weights (two E4M3 blocks) and feeds one MFMA per
-// activation block, as the GEMV above does; a block's sums run in the same order for any kMB.
-typedef __attribute__((address_space(3))) void GemvLds;
-constexpr int kRowBlockFrom = 4;                  // rows above which the row-block form runs
-constexpr int kChunkCols = 512;                   // activation columns a chunk
-constexpr int kXRowBytes = 2 * kChunkCols + 16;   // one activation row of a chunk, padded
-constexpr int kRowsAhead = 8;                     // macro steps of codes in flight a wave
+// The row-tile form (K % 128 == 0): a workgroup of 8 waves takes kTiles 16-row weight tiles, 32 rows
+// apart in one 128-row scale block, and splits K over its waves: wave w takes the 128-column steps w,
+// w + 8, .... Per step and tile a lane decodes its row's 32 weights (16 code bytes, two E4M3 blocks)
+// and feeds four MFMAs for each of kCols blocks of 16 activation rows, on the same columns of both
+// (column 128t + 32·(l/16) + 8q .. + 8 for MFMA q, as the GEMV above does). An activation piece
+// serves the kTiles tiles, and so does a scale load: the 16 bytes of a 128x4 tile's row hold the
+// scales of rows 32 apart. Two passes of kSteps steps' loads are in flight. Every load is in bounds
+// by itself: rows past N or M and steps past the wave's last read the last one, and nothing uses
+// what they bring. The waves' partial sums meet in LDS and are added in wave order; a wave's steps
+// do not depend on kSteps, kCols or kTiles, so a row's result does not depend on M.
+//
+// Bound: the activation reads through L2 and the loads' latency; the stream alone is 6 us of K=4096
+// N=14336's 11.3 at 5 rows. The decode is not (bf16's, twice the instructions, measures 0.2 us more).
+// fp16 activations decode by v_cvt_scalef32_pk_f16_fp4 and a packed fp16 multiply by the scale, both
+// exact (2 + 4 significant bits, 2^-10 .. 2688): one instruction a weight where the float32 way takes
+// two and a half. bf16 has no packed multiply and keeps it.
+constexpr int kTileWaves = 8;
+constexpr int kTilePolicy = 3;  // sc0 nt: each code byte is read once per call
 
-template <int N>
-__device__ __forceinline__ void gemv_vmcnt() {
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
+struct HalfPair {
+    f16x2n s;  // the two blocks' scales
+};
+
+template <bool kHalf>
+__device__ __forceinline__ auto block_scales(uint32_t b) {
+    if constexpr (kHalf) return HalfPair{__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(static_cast<int>(b), 1.0f, false)};
+    else return scales2(b);
 }
 
-// One wave's share of a chunk's activation rows: row r (r % 4 == wave) is one 1 KiB load.
-template <int kMB>
-__device__ __forceinline__ void gemv_chunk(__amdgpu_buffer_rsrc_t xr, uint8_t* slot, int chunk, int M, int K,
-                                           int wave, int lane) {
-    const int col = chunk * (2 * kChunkCols) + 16 * lane;  // byte within a row
-#pragma unroll
-    for (int j = 0; j < 4 * kMB; ++j) {
-        const int r = 4 * j + wave;
-        const uint32_t off = (r < M && col < 2 * K) ? static_cast<uint32_t>(r * 2 * K + col) : 0x80000000u;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (GemvLds*)(slot + r * kXRowBytes), 16, off, 0, 0, 0);
-    }
+// The eight weights of one code dword times block scale `which` of the pair.
+__device__ __forceinline__ i32x4 decode8(uint32_t word, HalfPair sc, int which) {
+    const int w = static_cast<int>(word);
+    const f16x2n s = which == 0 ? f16x2n{sc.s[0], sc.s[0]} : f16x2n{sc.s[1], sc.s[1]};
+    return i32x4{__builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 0) * s),
+                 __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 1) * s),
+                 __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 2) * s),
+                 __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 3) * s)};
 }
 
-template <bool kXHalf, bool kOutHalf, int kMB>
-__global__ __launch_bounds__(256) void nvfp4_rows_kernel(const uint16_t* __restrict__ x,
-                                                         const uint8_t* __restrict__ w,
-                                                         const uint8_t* __restrict__ scale,
-                                                         const float* __restrict__ scale_2,
-                                                         uint16_t* __restrict__ out, int M, int N, int K) {
-    constexpr int kSlot = 16 * kMB * kXRowBytes;
-    constexpr int kRing = kMB <= 2 ? 3 : 2;  // activation chunks in LDS (2 in flight when 3)
-    __shared__ __attribute__((aligned(16))) uint8_t xs[kRing * kSlot];
+__device__ __forceinline__ i32x4 decode8(uint32_t word, f32x2n sc, int which) {
+    return weights8<false>(word, sc[which]);
+}
+
+template <bool kXHalf, int kSteps, int kCols, int kTiles>
+__global__ __launch_bounds__(64 * kTileWaves) void nvfp4_tiles_kernel(
+    const uint16_t* x, const uint8_t* w, const uint8_t* scale, const float* scale_2, uint16_t* out,
+    int out_half, int M, int N, int K) {
+    // (Not __restrict__: the loads must stay in issue order.)
+    constexpr int kBlocks = kCols * kTiles;
+    static_assert(kTiles == 1 || kTiles == 2 || kTiles == 4, "scale loads of 4, 8 or 16 bytes");
+    __shared__ f32x4 part[kTileWaves][kBlocks][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const int n0 = blockIdx.x * 64 + 16 * wave;  // the wave's first weight row
-    const int row = n0 + (lane & 15);
-    const int sub = lane >> 4;
-    const int col_tiles = K / 64;
+    const int r = lane & 15, g = lane >> 4;
+    // The workgroup's first row: of its 128-row block, quarter `quarter` (of 32 rows; tile i is in
+    // quarter + i) and half of the quarter.
+    constexpr int kPer = 8 / kTiles;
+    const int in_block = blockIdx.x % kPer, quarter = in_block / 2 * kTiles;
+    const int n0 = 128 * (blockIdx.x / kPer) + 32 * quarter + 16 * (in_block & 1);
+    const int steps = K / 128, col_tiles = K / 64;
     const __amdgpu_buffer_rsrc_t wr = bounded_rsrc(w, static_cast<int64_t>(N) * (K / 2));
     const __amdgpu_buffer_rsrc_t sr = bounded_rsrc(scale, static_cast<int64_t>((N + 127) / 128 * 128) * col_tiles * 4);
     const __amdgpu_buffer_rsrc_t xr = bounded_rsrc(x, static_cast<int64_t>(M) * K * 2);
-    // Rows past N read past the codes' end (zeros).
-    const int64_t code_base = static_cast<int64_t>(row < N ? row : N) * (K / 2) + 16 * sub;
-    const int tile_row = (row >> 7) * col_tiles, in_tile = (row & 31) * 16 + ((row & 127) >> 5) * 4;
-    const int macro = K / 128, chunks = (macro + 3) / 4;
+    const float level = scale_2[0];
+    uint32_t code_at[kTiles], x_at[kCols];
+#pragma unroll
+    for (int i = 0; i < kTiles; ++i) code_at[i] = static_cast<uint32_t>(min(n0 + 32 * i + r, N - 1)) * static_cast<uint32_t>(K / 2) + 16 * g;
+#pragma unroll
+    for (int c = 0; c < kCols; ++c) x_at[c] = static_cast<uint32_t>(min(16 * c + r, M - 1)) * static_cast<uint32_t>(2 * K) + 64 * g;
+    // Scale block tile (n0 / 128, 2t + g/2), the 16 bytes of row n0 % 32 + r, from `quarter` on.
+    const uint32_t scale_at = static_cast<uint32_t>(n0 >> 7) * static_cast<uint32_t>(col_tiles * 512) + 512 * (g >> 1) + 16 * ((n0 & 31) + r) + 4 * quarter;
 
-    i32x4 code[kRowsAhead];
-    uint32_t sbyte[kRowsAhead];
-    auto load = [&](int t, int slot) {  // past the last step: zeros, never used
-        const bool live = t < macro;
-        code[slot] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(
-            wr, live ? static_cast<int>(code_base + 64 * t) : 0x7ffffff0, 0, 0));
-        const int b = 8 * t + 2 * sub;  // the first of its two blocks (even)
-        const int sidx = row < N && live ? ((tile_row + (b >> 2)) * 512 + in_tile + (b & 3)) : 0x7ffffff0;
-        sbyte[slot] = __builtin_amdgcn_raw_buffer_load_b16(sr, sidx, 0, 0);
+    struct Loads {
+        uint4 code[kSteps][kTiles];
+        uint32_t scale[kSteps][kTiles];  // the four bytes of the tile's column tile
+        i32x4 x[kSteps][kCols][4];
     };
-
-    f32x4 acc[kMB];
+    const int mine = (steps - wave + kTileWaves - 1) / kTileWaves;  // the wave's steps
+    auto issue = [&](int first, Loads& f) {
 #pragma unroll
-    for (int b = 0; b < kMB; ++b) acc[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    // Issue order, per chunk: its activation DMA, then 8 code and scale loads; so at chunk c's
-    // wait the loads issued after chunk c's DMA number 8 + (kRing - 2)·(4·kMB + 8).
-    gemv_chunk<kMB>(xr, xs, 0, M, K, wave, lane);
+        for (int j = 0; j < kSteps; ++j) {
+            const int t = min(wave + kTileWaves * min(first + j, max(mine - 1, 0)), steps - 1);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) load(t, t);
-    if constexpr (kRing == 3) gemv_chunk<kMB>(xr, xs + kSlot, 1, M, K, wave, lane);
+            for (int i = 0; i < kTiles; ++i)
+                f.code[j][i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wr, code_at[i], 64 * t, kTilePolicy));
+            if constexpr (kTiles == 4) {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b128(sr, scale_at, 1024 * t, 0);
 #pragma unroll
-    for (int t = 4; t < kRowsAhead; ++t) load(t, t);
-
-    // kRowsAhead / 4 chunks (the register window) an iteration, so that slots are static.
-    constexpr int kWindowChunks = kRowsAhead / 4;
-    for (int c0 = 0; c0 < chunks; c0 += kWindowChunks) {
+                for (int i = 0; i < 4; ++i) f.scale[j][i] = v[i];
+            } else if constexpr (kTiles == 2) {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b64(sr, scale_at, 1024 * t, 0);
+                f.scale[j][0] = v[0];
+                f.scale[j][1] = v[1];
+            } else {
+                f.scale[j][0] = __builtin_amdgcn_raw_buffer_load_b32(sr, scale_at, 1024 * t, 0);
+            }
 #pragma unroll
-        for (int h = 0; h < kWindowChunks; ++h) {
-            const int c = c0 + h;
-            // Chunk c landed (this wave's rows; the barrier makes every wave's visible), and
-            // every wave is done with chunk c - 1's slot, which takes chunk c + kRing - 1.
-            gemv_vmcnt<8 + (kRing - 2) * (4 * kMB + 8)>();
-            __syncthreads();
-            if (c >= chunks) break;
-            gemv_chunk<kMB>(xr, xs + ((c + kRing - 1) % kRing) * kSlot, c + kRing - 1, M, K, wave, lane);
-            const uint8_t* xc = xs + (c % kRing) * kSlot;
+            for (int c = 0; c < kCols; ++c)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int t = 4 * c + i, slot = 4 * h + i;
-                if (t < macro) {
-                    const f32x2n sc = scales2(sbyte[slot]);
-                    const float s0 = sc[0], s1 = sc[1];
+                for (int q = 0; q < 4; ++q)
+                    f.x[j][c][q] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, x_at[c] + 16 * q, 256 * t, 0));
+            asm volatile("" ::: "memory");
+        }
+    };
+    f32x4 acc[kTiles][kCols];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const i32x4 wq = weights8<kXHalf>(static_cast<uint32_t>(code[slot][q]), q < 2 ? s0 : s1);
+    for (int i = 0; i < kTiles; ++i)
 #pragma unroll
-                        for (int b = 0; b < kMB; ++b) {
-                            const i32x4 xv = *reinterpret_cast<const i32x4*>(
-                                xc + (16 * b + (lane & 15)) * kXRowBytes + 256 * i + 2 * (32 * sub + 8 * q));
-                            acc[b] = mfma16<kXHalf>(wq, xv, acc[b]);
-                        }
-                    }
+        for (int c = 0; c < kCols; ++c) acc[i][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto multiply = [&](int first, const Loads& f) {
+#pragma unroll
+        for (int j = 0; j < kSteps; ++j) {
+            if (first + j >= mine) break;  // uniform
+#pragma unroll
+            for (int i = 0; i < kTiles; ++i) {
+                const auto sc = block_scales<kXHalf>(f.scale[j][i] >> (16 * (g & 1)));
+                const uint32_t d[4] = {f.code[j][i].x, f.code[j][i].y, f.code[j][i].z, f.code[j][i].w};
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const i32x4 wq = decode8(d[q], sc, q / 2);
+#pragma unroll
+                    for (int c = 0; c < kCols; ++c) acc[i][c] = mfma16<kXHalf>(wq, f.x[j][c][q], acc[i][c]);
                 }
-                load(t + kRowsAhead, slot);
             }
         }
+    };
+    const int passes = (steps + kTileWaves * kSteps - 1) / (kTileWaves * kSteps);
+    Loads a;
+    issue(0, a);
+    // Two sets of loads where they fit the registers; else the other wave of the SIMD fills the wait.
+    constexpr bool kTwoSets = kSteps * (5 * kTiles + 16 * kCols) <= 72;
+    if (passes == 1) {
+        multiply(0, a);
+    } else if constexpr (!kTwoSets) {
+        multiply(0, a);
+        for (int p = 1; p < passes; ++p) {
+            issue(p * kSteps, a);
+            multiply(p * kSteps, a);
+        }
+    } else {
+        Loads b;
+        for (int p = 0; p < passes; p += 2) {
+            issue((p + 1) * kSteps, b);
+            multiply(p * kSteps, a);
+            issue((p + 2) * kSteps, a);
+            multiply((p + 1) * kSteps, b);
+        }
     }
-    gemv_vmcnt<0>();  // the zero loads past the end land before the wave ends
 
-    // D[i][m]: lane holds MFMA rows 4·(lane/16) + r of column m = lane % 16.
-    const float g = scale_2[0];
-    const int n = n0 + 4 * sub;
+    // D[i][m]: lane holds MFMA rows 4·(lane/16) + 0..3 of column m = lane % 16. Wave b adds block b's
+    // partial sums, in wave order.
 #pragma unroll
-    for (int b = 0; b < kMB; ++b) {
-        const int m = 16 * b + (lane & 15);
-        if (m >= M) continue;
+    for (int i = 0; i < kTiles; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            if (n + r < N) out[static_cast<int64_t>(m) * N + n + r] = narrow<kOutHalf>(acc[b][r] * g);
+        for (int c = 0; c < kCols; ++c) part[wave][i * kCols + c][lane] = acc[i][c];
+    __syncthreads();
+    const bool whole = N % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0;
+    for (int b = wave; b < kBlocks; b += kTileWaves) {
+        f32x4 sum = part[0][b][lane];
+#pragma unroll
+        for (int v = 1; v < kTileWaves; ++v) {
+            const f32x4 p = part[v][b][lane];
+            sum = f32x4{sum[0] + p[0], sum[1] + p[1], sum[2] + p[2], sum[3] + p[3]};
+        }
+        const int m = 16 * (b % kCols) + r, n = n0 + 32 * (b / kCols) + 4 * g;
+        if (m >= M || n >= N) continue;
+        uint16_t o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = out_half ? narrow<true>(sum[i] * level) : narrow<false>(sum[i] * level);
+        uint16_t* dst = out + static_cast<int64_t>(m) * N + n;
+        if (whole) {
+            *reinterpret_cast<uint2*>(dst) = make_uint2(o[0] | (static_cast<uint32_t>(o[1]) << 16), o[2] | (static_cast<uint32_t>(o[3]) << 16));
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (n + i < N) dst[i] = o[i];
+        }
     }
 }
 
@@ -466,9 +519,8 @@ hipError_t nvfp4_gemv(const void* x, bool x_half, const uint8_t* w, const uint8_
                       void* out, bool out_half, int M, int N, int K, hipStream_t s) {
     const auto* xp = static_cast<const uint16_t*>(x);
     auto* op = static_cast<uint16_t*>(out);
-    // More than 4 rows on a weight whose 64-row groups alone give 192 workgroups: the row-block
-    // kernel (the activation read once per workgroup); otherwise the K-split GEMV.
-    const bool rows = M > kRowBlockFrom && K % 128 == 0 && (N + 63) / 64 >= 192;
+    using T = std::true_type;
+    using F = std::false_type;
     // One or two rows of a short activation: the streaming form.
     if (M >= 1 && M <= kStreamRowsMax && K <= kStreamMaxK) {
         const int64_t lds = (static_cast<int64_t>(M) * 4096 + 1024) * ((K + 2047) / 2048);
@@ -481,34 +533,62 @@ hipError_t nvfp4_gemv(const void* x, bool x_half, const uint8_t* w, const uint8_
             constexpr bool kX = decltype(xh)::value, kO = decltype(oh)::value;
             return M == 1 ? stream(nvfp4_stream_kernel<kX, kO, 1>) : stream(nvfp4_stream_kernel<kX, kO, 2>);
         };
-        using T = std::true_type;
-        using F = std::false_type;
         if (x_half) return out_half ? by_rows(T{}, T{}) : by_rows(T{}, F{});
         return out_half ? by_rows(F{}, T{}) : by_rows(F{}, F{});
     }
+    // Whole 128-column steps: the row-tile form, as many 16-row tiles a workgroup as leave one
+    // workgroup a CU (us, graph replays over weights past the MALL, K-split or row-block form / this:
+    // K=4096 N=14336 M=5 14.7 / 11.3, M=16 15.4 / 13.7, M=64 29.7 / 24.5; K=3072 N=9216 M=24 24.9 /
+    // 16.0; K=14336 N=4096 M=2 14.9 / 12.7, M=64 73.5 / 60.7). Where a tile a workgroup is all there is
+    // (N <= 4096) nothing shares the activation, and 9..48 rows keep the K-split form, the same bits
+    // (K=3072 N=3072 M=40 13.3 / 15.8; K=14336 N=4096 M=16 21.1 / 21.5).
+    const int tiles = (N + 15) / 16, share = tiles > 512 ? 4 : tiles > 256 ? 2 : 1;
+    if (K % 128 == 0 && M >= 1 && (share > 1 || M <= 8 || M > 48)) {
+        auto tiled = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((N + 127) / 128 * (8 / share)), dim3(64 * kTileWaves), 0, s, xp, w, scale, scale_2, op, out_half, M, N, K);
+            return hipGetLastError();
+        };
+        // One step a pass, or all of a short K in one (K=4096 N=4096 M=5 6.3 us and 5.7; K=2048 N=6144
+        // M=7 5.9 and 5.1); longer passes of more tiles hold too many registers.
+        const int steps = K / 128;
+        auto by = [&](auto xh) {
+            constexpr bool kX = decltype(xh)::value;
+            const int cols = (M + 15) / 16;
+            if (share == 4) {
+                switch (cols) {
+                    case 1: return tiled(nvfp4_tiles_kernel<kX, 1, 1, 4>);
+                    case 2: return tiled(nvfp4_tiles_kernel<kX, 1, 2, 4>);
+                    case 3: return tiled(nvfp4_tiles_kernel<kX, 1, 3, 4>);
+                    default: return tiled(nvfp4_tiles_kernel<kX, 1, 4, 4>);
+                }
+            }
+            if (share == 2) {
+                switch (cols) {
+                    case 1: return steps <= 16 ? tiled(nvfp4_tiles_kernel<kX, 2, 1, 2>) : tiled(nvfp4_tiles_kernel<kX, 1, 1, 2>);
+                    case 2: return tiled(nvfp4_tiles_kernel<kX, 1, 2, 2>);
+                    case 3: return tiled(nvfp4_tiles_kernel<kX, 1, 3, 2>);
+                    default: return tiled(nvfp4_tiles_kernel<kX, 1, 4, 2>);
+                }
+            }
+            if (cols == 1) return steps <= 32 ? tiled(nvfp4_tiles_kernel<kX, 4, 1, 1>) : tiled(nvfp4_tiles_kernel<kX, 1, 1, 1>);
+            return tiled(nvfp4_tiles_kernel<kX, 1, 4, 1>);
+        };
+        return x_half ? by(T{}) : by(F{});
+    }
     auto go = [&](auto kernel) {
-        if (rows)
-            hipLaunchKernelGGL(kernel, dim3((N + 63) / 64), dim3(256), 0, s, xp, w, scale, scale_2, op, M, N, K);
-        else
-            hipLaunchKernelGGL(kernel, dim3((N + 127) / 128 * 8), dim3(64 * kGemvWaves), 0, s, xp, w, scale, scale_2, op, M, N, K);
+        hipLaunchKernelGGL(kernel, dim3((N + 127) / 128 * 8), dim3(64 * kGemvWaves), 0, s, xp, w, scale, scale_2, op, M, N, K);
         return hipGetLastError();
     };
     auto blocks = [&](auto xh, auto oh) {
         constexpr bool kX = decltype(xh)::value, kO = decltype(oh)::value;
-        switch ((M + 15) / 16 + (rows ? 4 : 0)) {
+        switch ((M + 15) / 16) {
             case 1: return go(nvfp4_gemv_kernel<kX, kO, 1>);
             case 2: return go(nvfp4_gemv_kernel<kX, kO, 2>);
             case 3: return go(nvfp4_gemv_kernel<kX, kO, 3>);
             case 4: return go(nvfp4_gemv_kernel<kX, kO, 4>);
-            case 5: return go(nvfp4_rows_kernel<kX, kO, 1>);
-            case 6: return go(nvfp4_rows_kernel<kX, kO, 2>);
-            case 7: return go(nvfp4_rows_kernel<kX, kO, 3>);
-            case 8: return go(nvfp4_rows_kernel<kX, kO, 4>);
             default: return hipErrorInvalidValue;
         }
     };
-    using T = std::true_type;
-    using F = std::false_type;
     if (x_half) return out_half ? blocks(T{}, T{}) : blocks(T{}, F{});
     return out_half ? blocks(F{}, T{}) : blocks(F{}, F{});
 }

@@ -53,6 +53,17 @@ def test_nvfp4_gemv_against_the_exact_product(dtype, m, n, k):
     _close(got, x.double() @ exact.double().t())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(3, 8, 128), (8, 4096, 4224), (7, 4104, 2048), (5, 4100, 2176), (16, 8192, 128), (17, 8200, 1024),
+                                   (33, 5128, 384), (48, 9216, 1152), (64, 12296, 640), (49, 520, 1152), (1, 264, 8192),
+                                   (2, 8328, 4224), (9, 4104, 4096)])  # fmt: skip
+def test_nvfp4_row_tiles_against_the_exact_product(dtype, m, n, k):
+    """The row-tile kernel at the edges of its dispatch: one, two and four weight tiles a workgroup
+    (256 tiles and one more, 512 and one more), one to four activation blocks, one pass and several
+    with waves that have no step, N off the tile and off a multiple of 4."""
+    test_nvfp4_gemv_against_the_exact_product(dtype, m, n, k)
+
+
 @pytest.mark.parametrize("n,sizes", [(4096, (3, 5, 16, 17, 33, 50)), (12288, (5, 9, 16, 17, 33, 50))])
 def test_nvfp4_gemv_rows_do_not_depend_on_m(n, sizes):
     """Within a kernel (the streaming form at 1 or 2 rows; the K-split GEMV; the row-block form
