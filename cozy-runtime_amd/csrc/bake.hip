@@ -10,11 +10,12 @@
 // under the seed, so a bake writes the bytes the reference's fused bake does for the same delta.
 // The delta is one float32 FMA chain per element over ranks 0, 1, ... from +0.
 //
-// A workgroup of 256 lanes takes a 64-row × 128-column tile: lane (rg = tid/16, cg = tid%16)
-// owns rows 4rg .. 4rg+3 and columns 4cg .. 4cg+3 and 64+4cg .. 64+4cg+3 (each 16-lane row of
-// a wave reads 256 contiguous bytes of LDS per rank). `up` (transposed) and `down` are staged
-// through LDS 32 ranks at a time. The hot part is the VALU: rank FMAs plus one Philox (ten
-// rounds, two 32x32→64-bit multiplies each) per element, against a few bytes of HBM.
+// A workgroup of 256 lanes takes a 64-row × 128-column tile, `up` and `down` staged through LDS
+// 32 ranks at a time. A few bytes of HBM an element against one Philox (ten rounds of two
+// 32x32→64-bit multiplies): the VALU is the bound. So `bake_kernel` takes its rank FMAs on the
+// float32 matrix unit (`Delta`); the other kernels keep them on the VALU (`tile_delta`): lane
+// (rg = tid/16, cg = tid%16) owns rows 4rg .. 4rg+3 and columns 4cg .. 4cg+3 and 64+4cg ..
+// 64+4cg+3 (each 16-lane row of a wave reads 256 contiguous bytes of LDS per rank).
 #include "common.h"
 #include "kernels.h"
 
@@ -22,6 +23,11 @@ namespace cozyq {
 namespace {
 
 constexpr int kTileRows = 64, kTileCols = 128, kRankChunk = 32, kBakeThreads = 256;
+
+// a ^ b ^ c in one instruction (the compiler leaves two; a draw takes 15 of these).
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+    return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+}
 
 // Philox4x32-10 (Salmon et al., SC'11) at counter (offset, 0, 0, 0) under key (k0, k1): the
 // first output word, Triton's `tl.randint`.
@@ -31,8 +37,8 @@ __device__ __forceinline__ uint32_t philox_word(uint32_t offset, uint32_t k0, ui
     for (int round = 0; round < 10; ++round) {
         const uint64_t pb = static_cast<uint64_t>(0xCD9E8D57u) * c2;
         const uint64_t pa = static_cast<uint64_t>(0xD2511F53u) * c0;
-        c0 = static_cast<uint32_t>(pb >> 32) ^ c1 ^ k0;
-        c2 = static_cast<uint32_t>(pa >> 32) ^ c3 ^ k1;
+        c0 = xor3(static_cast<uint32_t>(pb >> 32), c1, k0);
+        c2 = xor3(static_cast<uint32_t>(pa >> 32), c3, k1);
         c1 = static_cast<uint32_t>(pb);
         c3 = static_cast<uint32_t>(pa);
         k0 += 0x9E3779B9u;
@@ -146,6 +152,90 @@ __device__ __forceinline__ void tile_delta(float (&acc)[4][8], const float* __re
     }
 }
 
+// The same delta on v_mfma_f32_16x16x4_f32, which sums its four ranks as the same float32 FMA
+// chain (each product unrounded, subnormals kept: the GPU tests hold its bits to the oracle's
+// chain). The unit runs beside the VALU, which the draws keep busy: rank 32 is 32 of the ~97 VALU
+// instructions an element was. Columns are the MFMA's rows, so that lane (q = lane/16, n =
+// lane%16) of wave w owns row 16w + n and columns [64g + 16q, +16) for g = 0, 1, in acc[g][t][i] =
+// column 64g + 16q + 4t + i: tile t's MFMA row 4q + i is that column, and `down` lies in LDS in
+// the order in which one 16-byte read serves four tiles. Ranks past the last multiply +0 by −0,
+// which leaves every sum as it is, a −0 too.
+struct Delta {
+    static constexpr int kUpPitch = 36;  // rows 36 floats apart: a read's 16 rows x 4 ranks hit 64 banks
+    float up[kTileRows][kUpPitch];
+    float down[kRankChunk][kTileCols];
+};
+
+__device__ __forceinline__ void mfma_delta(f32x4 (&acc)[2][4], const float* __restrict__ up,
+                                           const float* __restrict__ down, int rows, int cols, int rank,
+                                           int row0, int col0, Delta& lds) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int q = lane >> 4, n = lane & 15;
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[g][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int r0 = 0; r0 < rank; r0 += kRankChunk) {
+        __syncthreads();  // the previous chunk is consumed
+        for (int e = tid; e < kRankChunk * kTileRows; e += kBakeThreads) {
+            const int k = e % kRankChunk, r = e / kRankChunk;
+            const int row = row0 + r, rk = r0 + k;
+            lds.up[r][k] = row < rows && rk < rank ? up[static_cast<int64_t>(row) * rank + rk] : 0.0f;
+        }
+        for (int e = tid; e < kRankChunk * kTileCols; e += kBakeThreads) {
+            const int c = e % kTileCols, k = e / kTileCols;
+            const int col = col0 + c, rk = r0 + k;
+            // Column 64g + 16a + 4t + b is row 4a + b of tile (g, t).
+            const int at = (c & 64) | (c & 48) | ((c & 3) << 2) | ((c >> 2) & 3);
+            lds.down[k][at] = rk >= rank ? -0.0f : col < cols ? down[static_cast<int64_t>(rk) * cols + col] : 0.0f;
+        }
+        __syncthreads();
+        const int steps = rank - r0 < kRankChunk ? (rank - r0 + 3) / 4 : kRankChunk / 4;
+        for (int s = 0; s < steps; ++s) {
+            const float u = lds.up[16 * wave + n][4 * s + q];
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                const f32x4 d = *reinterpret_cast<const f32x4*>(&lds.down[4 * s + q][64 * g + 4 * n]);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) acc[g][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[t], u, acc[g][t], 0, 0, 0);
+            }
+        }
+    }
+}
+
+// A lane's 32 deltas over its row's `unit`, in place, each RN(d / unit). Where unit and every delta
+// are far from the ends of the range, so that quotient and remainder are exact to scale, by the
+// row's reciprocal and one correction (as `div_rn`: 3 instructions, where a division is 10 and a
+// reciprocal); a lane with a zero, tiny, huge or infinite delta divides. A NaN is one either way.
+__device__ __forceinline__ void over_unit(f32x4 (&acc)[2][4], float unit) {
+    float most = 0.0f, least = 1.0f;
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                most = __builtin_fmaxf(most, __builtin_fabsf(acc[g][t][i]));
+                least = __builtin_fminf(least, __builtin_fabsf(acc[g][t][i]));
+            }
+    const bool near = unit >= 0x1p-40f && unit <= 0x1p40f && least >= 0x1p-60f && most <= 0x1p60f;
+    const float r = 1.0f / unit;
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            if (near) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float d = acc[g][t][i], quotient = d * r;
+                    acc[g][t][i] = __builtin_fmaf(__builtin_fmaf(-quotient, unit, d), r, quotient);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[g][t][i] = acc[g][t][i] / unit;
+            }
+}
+
 // Stored element types by form.
 template <int kForm> struct Stored;
 template <> struct Stored<kBakeBf16> { using T = uint16_t; };
@@ -189,8 +279,8 @@ struct Extra {
     float level, need_inv;
 };
 
-// One element of a `_bake_kernel` form: the stored value (its bits), the delta, the row's unit
-// (ROWWISE, INT8) or gain (plain, with kExtra), and the element's Philox counter → the new stored
+// One element of a `_bake_kernel` form: the stored value (its bits), the delta (on a kept ROWWISE
+// or INT8 scale already over the row's unit), the row's unit (ROWWISE, INT8) or gain (plain, with kExtra), and the element's Philox counter → the new stored
 // value. Without kExtra this is the fused law exactly; with it, plain rows are
 // round(round(v·gain) + delta) and every form can round to nearest.
 template <int kForm, bool kExtra>
@@ -224,12 +314,12 @@ __device__ __forceinline__ typename Stored<kForm>::T bake_one(typename Stored<kF
             // the delta, over the row's new scale.
             payload = (e4m3_sat(v) * unit + d) / fresh;
         } else {
-            payload = kExtra && x.no_delta ? e4m3_sat(v) : e4m3_sat(v) + d / unit;
+            payload = kExtra && x.no_delta ? e4m3_sat(v) : e4m3_sat(v) + d;
         }
         if (kExtra && x.nearest) return static_cast<uint8_t>(e4m3_nearest(payload));
         return static_cast<uint8_t>(e4m3_stochastic(payload, philox_word(at, k0, k1)));
     } else {
-        const float payload = kExtra && x.no_delta ? static_cast<float>(v) : static_cast<float>(v) + d / unit;
+        const float payload = kExtra && x.no_delta ? static_cast<float>(v) : static_cast<float>(v) + d;
         const float stored = kExtra && x.nearest ? __builtin_rintf(payload)
                                                  : __builtin_floorf(payload + uniform(philox_word(at, k0, k1)));
         return static_cast<int8_t>(__builtin_fminf(__builtin_fmaxf(stored, -127.0f), 127.0f));
@@ -245,8 +335,8 @@ __device__ __forceinline__ float with_more(float d, const Extra& x, int64_t at) 
     return d;
 }
 
-// kVec: cols % 4 == 0 and `data` aligned to four elements, so each lane's four-column group
-// moves as one load and one store.
+// kVec: cols % 4 == 0 and `data` aligned to four elements, so each lane's four-column groups
+// move as one load and one store each (all four of a 16-column run as one where cols has them).
 template <int kForm, bool kVec, bool kExtra>
 __global__ __launch_bounds__(kBakeThreads) void bake_kernel(typename Stored<kForm>::T* __restrict__ data,
                                                             const float* __restrict__ scale,
@@ -254,46 +344,78 @@ __global__ __launch_bounds__(kBakeThreads) void bake_kernel(typename Stored<kFor
                                                             const float* __restrict__ down, Extra x, int rows,
                                                             int cols, int rank, uint32_t seed) {
     using T = typename Stored<kForm>::T;
-    __shared__ float up_lds[kRankChunk][kTileRows];
-    __shared__ float down_lds[kRankChunk][kTileCols];
+    struct alignas(4 * sizeof(T)) Four { T v[4]; };
+    __shared__ __attribute__((aligned(16))) Delta lds;
     const int row0 = blockIdx.y * kTileRows, col0 = blockIdx.x * kTileCols;
-    float acc[4][8];
-    tile_delta(acc, up, down, rows, cols, rank, row0, col0, up_lds, down_lds);
-    const int rg = threadIdx.x >> 4, cg = threadIdx.x & 15;
+    f32x4 acc[2][4];
+    mfma_delta(acc, up, down, rows, cols, rank, row0, col0, lds);
+    const int lane = threadIdx.x & 63, q = lane >> 4;
+    const int row = row0 + 16 * (threadIdx.x >> 6) + (lane & 15);
+    if (row >= rows) return;
     const uint32_t k1 = (seed >> 31) ? 0xFFFFFFFFu : 0u;  // the int32 seed sign-extended
+    float unit = 1.0f, fresh = 1.0f;
+    if constexpr (kForm == kBakeRowwise || kForm == kBakeInt8) unit = scale[row];
+    else if (kExtra && x.gain) unit = x.gain[row];
+    if constexpr (kForm == kBakeRowwise) {
+        if (kExtra && x.rescale) fresh = x.rescale[row];
+    }
+    const int64_t line0 = static_cast<int64_t>(row) * cols;
+    if constexpr (kExtra) {
+        if (x.more) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = row0 + 4 * rg + i;
-        if (row >= rows) break;
-        float unit = 1.0f, fresh = 1.0f;
-        if constexpr (kForm == kBakeRowwise || kForm == kBakeInt8) unit = scale[row];
-        else if (kExtra && x.gain) unit = x.gain[row];
-        if constexpr (kForm == kBakeRowwise) {
-            if (kExtra && x.rescale) fresh = x.rescale[row];
+            for (int g = 0; g < 2; ++g)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int col = col0 + 64 * g + 16 * q + 4 * t + i;
+                        if (col < cols) acc[g][t][i] += x.more[line0 + col];
+                    }
         }
-        const int64_t line0 = static_cast<int64_t>(row) * cols;
-        T* line = data + line0;
-        const uint32_t line_at = static_cast<uint32_t>(static_cast<uint64_t>(row) * static_cast<uint64_t>(cols));
+    }
+    if constexpr (kForm == kBakeRowwise || kForm == kBakeInt8) {
+        if (!(kExtra && kForm == kBakeRowwise && x.rescale)) over_unit(acc, unit);
+    }
+    T* const line = data + line0;
+    const uint32_t line_at = static_cast<uint32_t>(static_cast<uint64_t>(row) * static_cast<uint64_t>(cols));
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int col = col0 + tile_col(cg, 4 * h);
-            if (col >= cols) continue;
-            if constexpr (kVec) {
-                struct alignas(4 * sizeof(T)) Four { T v[4]; };
-                Four four = *reinterpret_cast<const Four*>(line + col);
+    for (int g = 0; g < 2; ++g) {
+        const int col = col0 + 64 * g + 16 * q;
+        if constexpr (kVec) {
+            Four four[4];
+            const bool whole = col + 16 <= cols;
+            if (whole) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    four.v[e] = bake_one<kForm, kExtra>(four.v[e], with_more<kExtra>(acc[i][4 * h + e], x, line0 + col + e),
-                                                        unit, fresh, x, line_at + col + e, seed, k1);
-                *reinterpret_cast<Four*>(line + col) = four;
+                for (int t = 0; t < 4; ++t) four[t] = *reinterpret_cast<const Four*>(line + col + 4 * t);
             } else {
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (col + e < cols)
-                        line[col + e] = bake_one<kForm, kExtra>(
-                            line[col + e], with_more<kExtra>(acc[i][4 * h + e], x, line0 + col + e), unit, fresh,
-                            x, line_at + col + e, seed, k1);
+                for (int t = 0; t < 4; ++t)
+                    if (col + 4 * t < cols) four[t] = *reinterpret_cast<const Four*>(line + col + 4 * t);
+                    else four[t] = Four{};
             }
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    four[t].v[i] = bake_one<kForm, kExtra>(four[t].v[i], acc[g][t][i], unit, fresh, x,
+                                                           line_at + col + 4 * t + i, seed, k1);
+            if (whole) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) *reinterpret_cast<Four*>(line + col + 4 * t) = four[t];
+            } else {
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    if (col + 4 * t < cols) *reinterpret_cast<Four*>(line + col + 4 * t) = four[t];
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int c = col + 4 * t + i;
+                    if (c < cols)
+                        line[c] = bake_one<kForm, kExtra>(line[c], acc[g][t][i], unit, fresh, x, line_at + c, seed, k1);
+                }
         }
     }
 }

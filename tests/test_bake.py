@@ -541,6 +541,58 @@ def test_gpu_bake_int8_convrot_bit_exact(rows, cols, rank):
     assert np.array_equal(stored["weight"].cpu().numpy(), want)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", [ob.BF16, ob.F32, ob.ROWWISE, ob.INT8])
+@pytest.mark.parametrize("cols,rank", [(149, 1), (148, 3), (148, 4), (128, 5), (144, 31), (136, 36)])
+def test_gpu_bake_far_deltas_bit_exact(form, cols, rank):
+    """Deltas and row scales over most of float32's range, subnormals, both zeros and overflow among
+    them, at ranks about the matrix unit's four and the chunk's 32: the chain and the division by a
+    row's scale are the oracle's to the bit."""
+    from cozyq import prebuilt
+
+    rows = 70
+    print(f"bake far form={form} cols={cols} rank={rank}", flush=True)
+    data, scale, rng = _stored_for(form, rows, cols, 7 * rank + form)
+    if form == ob.F32:
+        data[:, ::3] = -0.0
+    up = rng.standard_normal((rows, rank))
+    up *= np.exp2(rng.integers(-75, 75, (rows, 1)).astype(np.float64))
+    down = rng.standard_normal((rank, cols))
+    down *= np.exp2(rng.integers(-70, 3, (1, cols)).astype(np.float64))
+    down[:, ::7] = -0.0
+    up, down = up.astype(np.float32), down.astype(np.float32)
+    up[::9] *= np.float32(2.0**-60)
+    up[1] = 0.0
+    if scale is not None:
+        scale = np.exp2(rng.uniform(-60, 60, scale.shape)).astype(np.float32)
+    seed = int(rng.integers(0, 1 << 31))
+    with np.errstate(all="ignore"):
+        want = ob.bake(form, data, scale, up, down, seed)
+    t = _torch_data(form, data).to(CUDA)
+    s = None if scale is None else torch.from_numpy(scale).to(CUDA)
+    prebuilt.library(0).bake(form, t, s, torch.from_numpy(up).to(CUDA), torch.from_numpy(down).to(CUDA), seed)
+    torch.cuda.synchronize()
+    assert np.array_equal(_bytes(t), want.view(np.uint8).reshape(rows, -1))
+
+
+@pytest.mark.gpu
+def test_gpu_bake_keeps_infinities_and_nans():
+    """A factor's infinity or NaN reaches the deltas of its row or column alone, ranks that pad the
+    last four included."""
+    from cozyq import prebuilt
+
+    rows, cols, rank = 33, 76, 6
+    rng = np.random.default_rng(5)
+    data = rng.standard_normal((rows, cols)).astype(np.float32)
+    up = rng.standard_normal((rows, rank)).astype(np.float32)
+    down = rng.standard_normal((rank, cols)).astype(np.float32)
+    up[3, 5], up[4, 0], down[2, 10] = np.inf, np.nan, -np.inf
+    want = data.astype(np.float64) + up.astype(np.float64) @ down.astype(np.float64)
+    t = torch.from_numpy(data.copy()).to(CUDA)
+    prebuilt.library(0).bake(ob.F32, t, None, torch.from_numpy(up).to(CUDA), torch.from_numpy(down).to(CUDA), 1)
+    np.testing.assert_allclose(t.cpu().numpy(), want, rtol=0, atol=2.0**-24 * 8 * 40)
+
+
 def _nvfp4_stored(rows: int, cols: int, rng):
     codes = rng.integers(0, 256, (rows, cols // 2), dtype=np.uint8)
     blocks = rng.integers(0x20, 0x48, (rows, cols // 16), dtype=np.uint8)  # E4M3 0.125 .. 2.0
