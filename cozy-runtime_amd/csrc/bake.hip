@@ -13,9 +13,11 @@
 // A workgroup of 256 lanes takes a 64-row × 128-column tile, `up` and `down` staged through LDS
 // 32 ranks at a time. A few bytes of HBM an element against one Philox (ten rounds of two
 // 32x32→64-bit multiplies): the VALU is the bound. So `bake_kernel` takes its rank FMAs on the
-// float32 matrix unit (`Delta`); the other kernels keep them on the VALU (`tile_delta`): lane
-// (rg = tid/16, cg = tid%16) owns rows 4rg .. 4rg+3 and columns 4cg .. 4cg+3 and 64+4cg ..
-// 64+4cg+3 (each 16-lane row of a wave reads 256 contiguous bytes of LDS per rank).
+// float32 matrix unit (`mfma_delta`: int8.convrot [12288, 3072] at rank 32, with the copy of the
+// stored weight, 110.6 → 103.7 us; the draw's 17 quarter-rate multiplies are what is left). The
+// other kernels keep them on the VALU (`tile_delta`): lane (rg = tid/16, cg = tid%16) owns rows
+// 4rg .. 4rg+3 and columns 4cg .. 4cg+3 and 64+4cg .. 64+4cg+3 (each 16-lane row of a wave reads
+// 256 contiguous bytes of LDS per rank).
 #include "common.h"
 #include "kernels.h"
 
