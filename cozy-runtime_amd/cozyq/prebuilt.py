@@ -769,8 +769,9 @@ class Prebuilt:
         scales = torch.empty(rows, dtype=torch.float32, device=x.device)
         scale, shift = self._table(scale, flat), self._table(shift, flat)
         first = shift if scale is None else scale
-        entries = (rows if first is None else first.shape[0]) or 1
-        if (shift is not None and shift.shape[0] != entries) or rows % entries:
+        entries = (rows or 1) if first is None else first.shape[0]
+        # (A table of no rows has no address, which the kernel takes for no table.)
+        if not entries or (shift is not None and shift.shape[0] != entries) or rows % entries:
             raise ValueError(f"{f.name}_quantize: modulation rows do not divide {rows} rows")
         code = self._lib.cozyq_quantize(
             self.index, f.fp8, flat.data_ptr(), self._half(flat.dtype), q.data_ptr(),

@@ -79,6 +79,21 @@ def test_operand_and_rows_messages(ops):
     assert ops._half(torch.float16) is True and ops._half(torch.bfloat16) is False
 
 
+@pytest.mark.parametrize("rows", [4, 0])
+def test_quantize_refuses_tables_that_do_not_cover_the_rows(rows):
+    """A modulation table of no rows is refused like one whose rows do not divide x's, whichever
+    of the two tables it is. (A library of index -1, the CPU's, reaches the check off the card.)"""
+    here = prebuilt.Prebuilt(torch, -1)
+    x = _aligned_empty(rows, 256, dtype=torch.bfloat16)
+    table = _aligned_empty(2, 256, dtype=torch.bfloat16)
+    none, three = table[:0], _aligned_empty(3, 256, dtype=torch.bfloat16)
+    refused = [(none, None), (none, none), (None, none), (table, none), (none, table), (table, table[:1])]
+    for scale, shift in refused + ([(three, None), (None, three)] if rows else []):
+        for quantize in (here.int8_quantize, here.fp8_quantize):
+            with pytest.raises(ValueError, match=f"modulation rows do not divide {rows} rows"):
+                quantize(x, scale, shift)
+
+
 def test_w4a8_weight_messages(ops):
     n, k = 16, 256
 
