@@ -94,6 +94,20 @@ class _FloatLane(_Lane):
         return product if leaf.bias is None else product + leaf.bias.to(product.dtype)
 
 
+def _read_parts(leaf: Any) -> tuple[Tensor, Tensor, Tensor | None]:
+    """`leaf`'s `data`, `scale` and `bias`, as its attributes say. A module's attribute that is a
+    buffer is found by a miss (1.7 us for the three, 0.2 from the buffers' table, of a call of 13), so a
+    leaf of the plain class reads its buffers by name where nothing else holds one of the names: a
+    parameter, a parametrization, a property or an attribute of its own."""
+    if type(leaf) is _module_class._cached:
+        own = leaf.__dict__
+        held = own["_buffers"]
+        if ("data" in held and "scale" in held and "bias" in held
+                and "data" not in own and "scale" not in own and "bias" not in own):  # fmt: skip
+            return read(held["data"]), read(held["scale"]), read(held["bias"])
+    return read(leaf.data), read(leaf.scale), read(leaf.bias)
+
+
 class _QuantizedLane(_Lane):
     """The 8-bit leaves (rule L4): a producer's operand goes straight to the GEMM; up to
     `few` rows with no operand take the op's one-launch linear; otherwise the operand handed
@@ -111,15 +125,11 @@ class _QuantizedLane(_Lane):
     def quantize(self, torch: Any, x: Tensor) -> PreQuantized | None:
         return int8_linear.quantize(torch, x)
 
-    # (The buffers by name: a module's attribute miss costs more than reading all three.)
     def gemm(self, torch, leaf, operand, out_dtype, out):
-        held = leaf._buffers
-        return int8_linear.gemm(torch, operand, read(held["data"]), read(held["scale"]), read(held["bias"]),
-                                out_dtype, out)  # fmt: skip
+        return int8_linear.gemm(torch, operand, *_read_parts(leaf), out_dtype, out)
 
     def linear(self, torch, leaf, x, out_dtype):
-        held = leaf._buffers
-        return int8_linear.linear(torch, x, read(held["data"]), read(held["scale"]), read(held["bias"]), out_dtype)
+        return int8_linear.linear(torch, x, *_read_parts(leaf), out_dtype)
 
     def run(self, torch, leaf, x, prequantized, out):
         if isinstance(x, PreQuantized):
@@ -144,13 +154,10 @@ class _Fp8Lane(_QuantizedLane):
         return fp8_linear.quantize(torch, x)
 
     def gemm(self, torch, leaf, operand, out_dtype, out):
-        held = leaf._buffers
-        return fp8_linear.gemm(torch, operand, read(held["data"]), read(held["scale"]), read(held["bias"]),
-                               out_dtype, out)  # fmt: skip
+        return fp8_linear.gemm(torch, operand, *_read_parts(leaf), out_dtype, out)
 
     def linear(self, torch, leaf, x, out_dtype):
-        held = leaf._buffers
-        return fp8_linear.linear(torch, x, read(held["data"]), read(held["scale"]), read(held["bias"]), out_dtype)
+        return fp8_linear.linear(torch, x, *_read_parts(leaf), out_dtype)
 
 
 class _W4a8Lane(_QuantizedLane):

@@ -164,6 +164,63 @@ def test_fp8_and_svdq_leaves_refuse_off_gpu():
         sv(torch.randn(2, 64, dtype=torch.bfloat16))
 
 
+def _bias_as_parameter(leaf, other):
+    leaf.bias = torch.nn.Parameter(other["bias"])
+
+
+def _data_as_parameter(leaf, other):
+    del leaf.data
+    leaf.register_parameter("data", torch.nn.Parameter(other["data"], requires_grad=False))
+
+
+def _scale_parametrized(leaf, other):
+    class Other(torch.nn.Module):
+        def forward(self, scale):
+            return other["scale"]
+
+    torch.nn.utils.parametrize.register_parametrization(leaf, "scale", Other())
+
+
+def _scale_as_property(leaf, other):
+    leaf.__class__ = type("Sub", (type(leaf),), {"scale": property(lambda self: other["scale"])})
+
+
+def _data_of_its_own(leaf, other):
+    leaf.__dict__["data"] = other["data"]
+
+
+def _bias_replaced(leaf, other):
+    leaf.bias = other["bias"]
+
+
+@pytest.mark.parametrize("change", [_bias_as_parameter, _data_as_parameter, _scale_parametrized, _scale_as_property,
+                                    _data_of_its_own, _bias_replaced])  # fmt: skip
+@pytest.mark.parametrize("provider,op", [(leaves.Int8ConvRotNativeLeaf, "int8_linear"),
+                                         (leaves.RowwiseNativeLeaf, "fp8_linear")])  # fmt: skip
+def test_8_bit_leaves_read_their_parts_as_attributes_say(monkeypatch, provider, op, change):
+    """The int8 and fp8 leaves hand their op the weight, scale and bias their attributes answer,
+    whether a name is still a buffer or has become a parameter, a parametrization, a property or an
+    attribute of the instance."""
+    code = torch.int8 if op == "int8_linear" else torch.float8_e4m3fn
+    leaf = provider().leaf(torch, {"weight": torch.zeros(8, 256).to(code), "scale": torch.ones(8)},
+                           _Linear(8, 256, True), torch.bfloat16)  # fmt: skip
+    other = {"data": torch.ones(8, 256).to(code), "scale": torch.full((8,), 2.0), "bias": torch.full((8,), 3.0)}
+    change(leaf, other)
+    seen = []
+    module = getattr(leaves, op)
+    monkeypatch.setattr(module, "linear", lambda torch, x, *parts: seen.append(parts[:3]) or x)
+    monkeypatch.setattr(module, "gemm", lambda torch, operand, *parts: seen.append(parts[:3]) or operand.payload)
+    x = torch.zeros(1, 256, dtype=torch.bfloat16)
+    leaf(x)
+    leaf(operands.PreQuantized(x.to(code), torch.ones(1), (1, 256), leaf.operand))
+    for data, scale, bias in seen:
+        assert torch.equal(data.float(), leaf.data.float()) and torch.equal(scale, leaf.scale)
+        assert torch.equal(bias, leaf.bias)
+    changed = change.__name__.split("_")[1]
+    got = dict(zip(("data", "scale", "bias"), seen[0]))
+    assert len(seen) == 2 and torch.equal(got[changed].float(), other[changed].float())
+
+
 def test_mx_leaf_untiles_cublas_scales():
     gen = torch.Generator().manual_seed(3)
     n, k = 136, 256
