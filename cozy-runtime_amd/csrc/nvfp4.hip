@@ -542,8 +542,10 @@ hipError_t nvfp4_gemv(const void* x, bool x_half, const uint8_t* w, const uint8_
     // 16.0; K=14336 N=4096 M=2 14.9 / 12.7, M=64 73.5 / 60.7). Where a tile a workgroup is all there is
     // (N <= 4096) nothing shares the activation, and 9..48 rows keep the K-split form, the same bits
     // (K=3072 N=3072 M=40 13.3 / 15.8; K=14336 N=4096 M=16 21.1 / 21.5).
+    // Scales that don't start at a dword keep the K-split form too, which reads them two bytes at a time.
     const int tiles = (N + 15) / 16, share = tiles > 512 ? 4 : tiles > 256 ? 2 : 1;
-    if (K % 128 == 0 && M >= 1 && (share > 1 || M <= 8 || M > 48)) {
+    const bool dwords = (reinterpret_cast<uintptr_t>(scale) & 3) == 0;
+    if (dwords && K % 128 == 0 && M >= 1 && (share > 1 || M <= 8 || M > 48)) {
         auto tiled = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3((N + 127) / 128 * (8 / share)), dim3(64 * kTileWaves), 0, s, xp, w, scale, scale_2, op, out_half, M, N, K);
             return hipGetLastError();

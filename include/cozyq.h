@@ -301,9 +301,10 @@ int cozyq_decode_svdq(int device, const uint8_t* w, const uint8_t* scale, int ti
  *   out[m, n] = round((Σ_k x[m, k] · (e2m1[n, k] · scale[n, k/16])) · scale_2), float32 sums.
  * w [N, K/2] E2M1 codes, element 2k in the low nibble; scale E4M3 in cuBLAS's 128x4 tiles over
  * [N, K/16] (the leaf's resident layout); scale_2 one float32. x [M, K] bf16 or fp16 (x_half),
- * 16-byte aligned; out [M, N] bf16 or fp16. 0 ≤ M ≤ 64, K % 32 == 0. With K % 128 == 0 a row-tile
- * kernel runs for more than 4096 outputs, and up to 8 and past 48 rows of fewer (1 and 2 rows with
- * K <= 4096 have a streaming kernel); within each kernel a row's result does not depend on M. */
+ * 16-byte aligned; out [M, N] bf16 or fp16. 0 ≤ M ≤ 64, K % 32 == 0. With K % 128 == 0 and `scale`
+ * at a 4-byte address a row-tile kernel runs for more than 4096 outputs, and up to 8 and past 48 rows
+ * of fewer (1 and 2 rows with K <= 4096 have a streaming kernel); within each kernel a row's result
+ * does not depend on M. */
 int cozyq_nvfp4_gemv(int device, const void* x, int x_half, const uint8_t* w, const uint8_t* scale,
                      const float* scale_2, void* out, int out_half, int M, int N, int K, void* stream);
 

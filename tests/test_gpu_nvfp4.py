@@ -64,6 +64,28 @@ def test_nvfp4_row_tiles_against_the_exact_product(dtype, m, n, k):
     test_nvfp4_gemv_against_the_exact_product(dtype, m, n, k)
 
 
+@pytest.mark.parametrize("skip", [2, 4, 8])
+@pytest.mark.parametrize("m,n,k", [(5, 12296, 640), (7, 4104, 1152), (3, 264, 256)])
+def test_nvfp4_gemv_takes_scales_off_their_alignment(m, n, k, skip):
+    """The block scales at an address that is no multiple of the row-tile kernel's 16-, 8- and 4-byte
+    loads: from a dword on that kernel reads them, at half of one the K-split form; the same bits as at
+    an aligned address."""
+    from cozyq import prebuilt
+
+    codes, _, blocked, second, exact = _weight(n, k, m + n)
+    x = torch.randn(m, k, generator=torch.Generator().manual_seed(k)).to(torch.bfloat16)
+    ops = prebuilt.library(0)
+    flat = blocked.reshape(-1)
+    moved = torch.zeros(flat.numel() + 16, dtype=torch.uint8, device=CUDA)[skip : skip + flat.numel()]
+    moved.copy_(flat)
+    assert moved.data_ptr() % 16 == skip
+    args = x.to(CUDA), codes.to(CUDA)
+    want = ops.nvfp4_gemv(*args, blocked.to(CUDA), second.to(CUDA), torch.bfloat16)
+    got = ops.nvfp4_gemv(*args, moved.view(blocked.shape), second.to(CUDA), torch.bfloat16)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    _close(got, x.double() @ exact.double().t())
+
+
 @pytest.mark.parametrize("n,sizes", [(4096, (3, 5, 16, 17, 33, 50)), (12288, (5, 9, 16, 17, 33, 50))])
 def test_nvfp4_gemv_rows_do_not_depend_on_m(n, sizes):
     """Within a kernel (the streaming form at 1 or 2 rows; the K-split GEMV; the row-block form
