@@ -691,7 +691,14 @@ __device__ __forceinline__ Int8Epilogue int8_epilogue(const float* xs, const flo
     e.bias = i32x2{0, 0};
     if (bias != nullptr) {
         const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(bias), 0, 2 * N, 0x00020000);
-        e.bias = __builtin_bit_cast(i32x2, __builtin_amdgcn_raw_buffer_load_b64(br, 2 * n, 0, 0));
+        if ((reinterpret_cast<uintptr_t>(bias) & 3) == 0) {  // uniform; a view may start at half a dword
+            e.bias = __builtin_bit_cast(i32x2, __builtin_amdgcn_raw_buffer_load_b64(br, 2 * n, 0, 0));
+        } else {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                e.bias[i] = __builtin_amdgcn_raw_buffer_load_b16(br, 2 * n + 4 * i, 0, 0) |
+                            (static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b16(br, 2 * n + 4 * i + 2, 0, 0)) << 16);
+        }
     }
     return e;
 }
@@ -1055,7 +1062,8 @@ hipError_t gemm_w4a8_narrow(const int8_t* q, const float* xs, const uint8_t* cod
         return bias ? launch_w4a8_decode<false, true>(q, xs, codes, w4, ws, bias, out, M, N, K, s)
                     : launch_w4a8_decode<false, false>(q, xs, codes, w4, ws, bias, out, M, N, K, s);
     }
-    if (config < 0 && M <= kW4RowsMax && (M <= 32 || K >= kW4RowsK)) {
+    // (A lane's two group scales come in one load, so an odd address keeps the narrow tiles' bytes.)
+    if (config < 0 && M <= kW4RowsMax && (M <= 32 || K >= kW4RowsK) && (reinterpret_cast<uintptr_t>(group_scale) & 1) == 0) {
         const W4 w4{group_scale, codebook};
         switch ((M + 15) / 16) {
             case 1: return launch_w4a8_rows<1>(q, xs, codes, w4, ws, bias, out, out_half, M, N, K, s);

@@ -1026,6 +1026,23 @@ def test_w4a8_row_tiles_bit_exact(ops, shape):
     assert torch.equal(got, laws.int8_linear(x, levels, scale, b, torch.bfloat16)[:rows])
 
 
+@pytest.mark.parametrize("shape", [(3, 136, 1024), (16, 4104, 2048), (40, 264, 1024), (64, 12296, 1024)],
+                         ids=lambda s: "x".join(map(str, s)))  # fmt: skip
+def test_w4a8_row_tiles_take_a_bias_off_its_alignment(ops, shape):
+    """A bias that is a view from an odd element on (a part of a fused one): the row-tile kernel's
+    outputs are those of the same values at an aligned address, bit for bit."""
+    m, n, k = shape
+    w, _, _ = _w4a8(n, k, 5 + m, True)
+    gen = torch.Generator().manual_seed(m)
+    q, s = ops.int8_quantize(torch.randn(m, k, generator=gen).to(torch.bfloat16).to(DEV))
+    for dtype in (torch.bfloat16, torch.float16):
+        fused = torch.randn(n + 8, generator=gen).to(dtype).to(DEV)
+        for skip in (1, 2, 3):
+            view = fused[skip : skip + n]
+            assert view.data_ptr() % 8 == 2 * skip
+            assert torch.equal(ops.w4a8_gemm(q, s, w, view, dtype), ops.w4a8_gemm(q, s, w, view.clone(), dtype))
+
+
 # ------------------------------------------------------------------------ MXFP8 lane
 
 
