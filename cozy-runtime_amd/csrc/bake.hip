@@ -14,10 +14,12 @@
 // 32 ranks at a time. A few bytes of HBM an element against one Philox (ten rounds of two
 // 32x32→64-bit multiplies): the VALU is the bound. So `bake_kernel` takes its rank FMAs on the
 // float32 matrix unit (`mfma_delta`: int8.convrot [12288, 3072] at rank 32, with the copy of the
-// stored weight, 110.6 → 103.7 us; the draw's 17 quarter-rate multiplies are what is left). The
+// stored weight, 110.6 → 100.3 us; the draw's 17 quarter-rate multiplies are what is left). The
 // other kernels keep them on the VALU (`tile_delta`): lane (rg = tid/16, cg = tid%16) owns rows
 // 4rg .. 4rg+3 and columns 4cg .. 4cg+3 and 64+4cg .. 64+4cg+3 (each 16-lane row of a wave reads
 // 256 contiguous bytes of LDS per rank).
+#include <type_traits>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -154,20 +156,30 @@ __device__ __forceinline__ void tile_delta(float (&acc)[4][8], const float* __re
     }
 }
 
+// How a wave's 16 rows and the tile's 128 columns fall to its lanes (q = lane/16, n = lane%16), for
+// `mfma_delta`'s acc[g][t][i], g = 0, 1, t = 0..3, i = 0..3:
+//   kRuns     row n, column 64g + 16q + 4t + i: 16 consecutive columns a lane and g, one 16-byte
+//             access of bytes, two of halves;
+//   kLanes    row 4q + i, column 64g + 4n + t: four consecutive columns a lane, and sixteen lanes on
+//             whole lines of one row;
+//   kColumns  row 4q + i, column 64g + 16t + n: sixteen lanes on consecutive columns, for rows that
+//             are read and written an element at a time (off-alignment, or columns % 4).
+enum BakeOrder { kRuns, kLanes, kColumns };
+
 // The same delta on v_mfma_f32_16x16x4_f32, which sums its four ranks as the same float32 FMA
 // chain (each product unrounded, subnormals kept: the GPU tests hold its bits to the oracle's
 // chain). The unit runs beside the VALU, which the draws keep busy: rank 32 is 32 of the ~97 VALU
-// instructions an element was. Columns are the MFMA's rows, so that lane (q = lane/16, n =
-// lane%16) of wave w owns row 16w + n and columns [64g + 16q, +16) for g = 0, 1, in acc[g][t][i] =
-// column 64g + 16q + 4t + i: tile t's MFMA row 4q + i is that column, and `down` lies in LDS in
-// the order in which one 16-byte read serves four tiles. Ranks past the last multiply +0 by −0,
-// which leaves every sum as it is, a −0 too.
+// instructions an element was. Columns are the MFMA's rows and rows its columns, so that a lane's
+// four results are consecutive columns (kColumns: the other way round). `down` lies in LDS in the
+// order in which one 16-byte read serves four tiles. Ranks past the last multiply +0 by −0, which
+// leaves every sum as it is, a −0 too.
 struct Delta {
     static constexpr int kUpPitch = 36;  // rows 36 floats apart: a read's 16 rows x 4 ranks hit 64 banks
     float up[kTileRows][kUpPitch];
     float down[kRankChunk][kTileCols];
 };
 
+template <BakeOrder kOrder>
 __device__ __forceinline__ void mfma_delta(f32x4 (&acc)[2][4], const float* __restrict__ up,
                                            const float* __restrict__ down, int rows, int cols, int rank,
                                            int row0, int col0, Delta& lds) {
@@ -187,8 +199,10 @@ __device__ __forceinline__ void mfma_delta(f32x4 (&acc)[2][4], const float* __re
         for (int e = tid; e < kRankChunk * kTileCols; e += kBakeThreads) {
             const int c = e % kTileCols, k = e / kTileCols;
             const int col = col0 + c, rk = r0 + k;
-            // Column 64g + 16a + 4t + b is row 4a + b of tile (g, t).
-            const int at = (c & 64) | (c & 48) | ((c & 3) << 2) | ((c >> 2) & 3);
+            // kRuns: column 64g + 16a + 4t + b is row 4a + b of tile (g, t).
+            const int at = kOrder == kRuns    ? (c & 64) | (c & 48) | ((c & 3) << 2) | ((c >> 2) & 3)
+                           : kOrder == kLanes ? c
+                                              : (c & 64) | ((c & 15) << 2) | ((c >> 4) & 3);
             lds.down[k][at] = rk >= rank ? -0.0f : col < cols ? down[static_cast<int64_t>(rk) * cols + col] : 0.0f;
         }
         __syncthreads();
@@ -199,24 +213,29 @@ __device__ __forceinline__ void mfma_delta(f32x4 (&acc)[2][4], const float* __re
             for (int g = 0; g < 2; ++g) {
                 const f32x4 d = *reinterpret_cast<const f32x4*>(&lds.down[4 * s + q][64 * g + 4 * n]);
 #pragma unroll
-                for (int t = 0; t < 4; ++t) acc[g][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[t], u, acc[g][t], 0, 0, 0);
+                for (int t = 0; t < 4; ++t)
+                    acc[g][t] = kOrder == kRuns ? __builtin_amdgcn_mfma_f32_16x16x4f32(d[t], u, acc[g][t], 0, 0, 0)
+                                                : __builtin_amdgcn_mfma_f32_16x16x4f32(u, d[t], acc[g][t], 0, 0, 0);
             }
         }
     }
 }
 
-// A lane's 32 deltas over its row's `unit`, in place, each RN(d / unit). Where unit and every delta
-// are far from the ends of the range, so that quotient and remainder are exact to scale, by the
-// row's reciprocal and one correction (as `div_rn`: 3 instructions, where a division is 10 and a
-// reciprocal); a lane with a zero, tiny, huge or infinite delta divides. A NaN is one either way.
+// Deltas of one row over its `unit`, in place, each RN(d / unit): all 32 of a lane, or the eight at
+// i = kOnly. Where unit and every delta are far from the ends of the range, so that quotient and
+// remainder are exact to scale, by the row's reciprocal and one correction (as `div_rn`: 3
+// instructions, where a division is 10 and a reciprocal); a lane with a zero, tiny, huge or infinite
+// delta divides. A NaN is one either way.
+template <int kOnly = -1>
 __device__ __forceinline__ void over_unit(f32x4 (&acc)[2][4], float unit) {
+    constexpr int kFirst = kOnly < 0 ? 0 : kOnly, kEnd = kOnly < 0 ? 4 : kOnly + 1;
     float most = 0.0f, least = 1.0f;
 #pragma unroll
     for (int g = 0; g < 2; ++g)
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+            for (int i = kFirst; i < kEnd; ++i) {
                 most = __builtin_fmaxf(most, __builtin_fabsf(acc[g][t][i]));
                 least = __builtin_fminf(least, __builtin_fabsf(acc[g][t][i]));
             }
@@ -228,13 +247,13 @@ __device__ __forceinline__ void over_unit(f32x4 (&acc)[2][4], float unit) {
         for (int t = 0; t < 4; ++t)
             if (near) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
+                for (int i = kFirst; i < kEnd; ++i) {
                     const float d = acc[g][t][i], quotient = d * r;
                     acc[g][t][i] = __builtin_fmaf(__builtin_fmaf(-quotient, unit, d), r, quotient);
                 }
             } else {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) acc[g][t][i] = acc[g][t][i] / unit;
+                for (int i = kFirst; i < kEnd; ++i) acc[g][t][i] = acc[g][t][i] / unit;
             }
 }
 
@@ -337,30 +356,124 @@ __device__ __forceinline__ float with_more(float d, const Extra& x, int64_t at) 
     return d;
 }
 
-// kVec: cols % 4 == 0 and `data` aligned to four elements, so each lane's four-column groups
-// move as one load and one store each (all four of a 16-column run as one where cols has them).
-template <int kForm, bool kVec, bool kExtra>
-__global__ __launch_bounds__(kBakeThreads) void bake_kernel(typename Stored<kForm>::T* __restrict__ data,
-                                                            const float* __restrict__ scale,
-                                                            const float* __restrict__ up,
-                                                            const float* __restrict__ down, Extra x, int rows,
-                                                            int cols, int rank, uint32_t seed) {
+// A row's unit (ROWWISE, INT8) or gain (plain, with kExtra), and its new scale where it takes one.
+template <int kForm, bool kExtra>
+__device__ __forceinline__ float2 row_units(const float* scale, const Extra& x, int row) {
+    float2 u = make_float2(1.0f, 1.0f);
+    if constexpr (kForm == kBakeRowwise || kForm == kBakeInt8) u.x = scale[row];
+    else if (kExtra && x.gain) u.x = x.gain[row];
+    if constexpr (kForm == kBakeRowwise) {
+        if (kExtra && x.rescale) u.y = x.rescale[row];
+    }
+    return u;
+}
+
+// kOrder kColumns reads and writes an element at a time; the others take cols % 4 == 0 and `data`
+// aligned to four elements, and move a lane's four consecutive columns as one load and one store
+// (kRuns: all four groups of a 16-column run as one where cols has them). The forms of bytes take
+// kRuns, the wider ones kLanes: a wave's access covers 16 rows in the first and 4 in the second, so
+// that wide elements come in whole lines ([8192, 12288] at rank 8, us on the VALU / as runs / as lanes:
+// float32 183 / 212 / 163, fp16 130 / 144 / 90, bf16 196 / 171 / 155; int8 207 / 162 / 164). Columns
+// an element at a time: [8192, 3074] at rank 8 fp16 75 on the VALU, 143 as runs, 43 as columns. Six
+// waves a SIMD where a lane reads ahead least: a tile's staging and its round trip to the weight hide
+// behind the others' draws.
+template <int kForm, BakeOrder kOrder>
+struct BakeShape {
+    // Rows of a lane that are in flight at once, and waves a SIMD.
+    static constexpr int kBatch = kOrder == kLanes && kForm == kBakeF32 ? 2 : 4;
+    static constexpr int kWaves = kOrder == kColumns ? 4 : kOrder == kLanes && kForm != kBakeF32 ? 5 : 6;
+};
+
+template <int kForm, BakeOrder kOrder, bool kExtra>
+__global__ __launch_bounds__(kBakeThreads, (BakeShape<kForm, kOrder>::kWaves)) void bake_kernel(
+    typename Stored<kForm>::T* __restrict__ data, const float* __restrict__ scale, const float* __restrict__ up,
+    const float* __restrict__ down, Extra x, int rows, int cols, int rank, uint32_t seed) {
     using T = typename Stored<kForm>::T;
     struct alignas(4 * sizeof(T)) Four { T v[4]; };
     __shared__ __attribute__((aligned(16))) Delta lds;
     const int row0 = blockIdx.y * kTileRows, col0 = blockIdx.x * kTileCols;
-    f32x4 acc[2][4];
-    mfma_delta(acc, up, down, rows, cols, rank, row0, col0, lds);
-    const int lane = threadIdx.x & 63, q = lane >> 4;
-    const int row = row0 + 16 * (threadIdx.x >> 6) + (lane & 15);
-    if (row >= rows) return;
+    const int lane = threadIdx.x & 63, q = lane >> 4, n = lane & 15;
+    const int wave_row = row0 + 16 * (threadIdx.x >> 6);
     const uint32_t k1 = (seed >> 31) ? 0xFFFFFFFFu : 0u;  // the int32 seed sign-extended
-    float unit = 1.0f, fresh = 1.0f;
-    if constexpr (kForm == kBakeRowwise || kForm == kBakeInt8) unit = scale[row];
-    else if (kExtra && x.gain) unit = x.gain[row];
-    if constexpr (kForm == kBakeRowwise) {
-        if (kExtra && x.rescale) fresh = x.rescale[row];
+    constexpr bool kScaled = kForm == kBakeRowwise || kForm == kBakeInt8;
+    const bool divides = kScaled && !(kExtra && kForm == kBakeRowwise && x.rescale);
+    f32x4 acc[2][4];
+    if constexpr (kOrder != kRuns) {
+        constexpr int kBatch = BakeShape<kForm, kOrder>::kBatch;
+        // A batch of rows is read before it is worked on, and its draws made before a store: one memory
+        // round trip a batch, and many draws in flight, where a test around each element runs one.
+        mfma_delta<kOrder>(acc, up, down, rows, cols, rank, row0, col0, lds);
+        auto column = [&](int g, int t) { return col0 + 64 * g + (kOrder == kLanes ? 4 * n + t : 16 * t + n); };
+        auto batch = [&](auto from) {
+            constexpr int kFrom = decltype(from)::value;
+            Four value[kBatch][2];
+            float2 u[kBatch];
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j) {
+                const int row = min(wave_row + 4 * q + kFrom + j, rows - 1);
+                u[j] = row_units<kForm, kExtra>(scale, x, row);
+                const T* const line = data + static_cast<int64_t>(row) * cols;
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    if constexpr (kOrder == kLanes) {
+                        value[j][g] = *reinterpret_cast<const Four*>(line + min(column(g, 0), cols - 4));
+                    } else {
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) value[j][g].v[t] = line[min(column(g, t), cols - 1)];
+                    }
+                }
+            }
+            auto one_row = [&](auto index) {
+                constexpr int j = decltype(index)::value, i = kFrom + j;
+                const int row = wave_row + 4 * q + i;
+                const int64_t line0 = static_cast<int64_t>(row) * cols;
+                const uint32_t line_at = static_cast<uint32_t>(static_cast<uint64_t>(row) * static_cast<uint64_t>(cols));
+                if constexpr (kExtra) {
+                    if (x.more && row < rows)
+#pragma unroll
+                        for (int g = 0; g < 2; ++g)
+#pragma unroll
+                            for (int t = 0; t < 4; ++t)
+                                if (column(g, t) < cols) acc[g][t][i] += x.more[line0 + column(g, t)];
+                }
+                if (divides) over_unit<i>(acc, u[j].x);
+#pragma unroll
+                for (int g = 0; g < 2; ++g)
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        value[j][g].v[t] = bake_one<kForm, kExtra>(value[j][g].v[t], acc[g][t][i], u[j].x, u[j].y, x,
+                                                                   line_at + column(g, t), seed, k1);
+            };
+            one_row(std::integral_constant<int, 0>{});
+            one_row(std::integral_constant<int, 1>{});
+            if constexpr (kBatch == 4) {
+                one_row(std::integral_constant<int, 2>{});
+                one_row(std::integral_constant<int, 3>{});
+            }
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j) {
+                const int row = wave_row + 4 * q + kFrom + j;
+                T* const line = data + static_cast<int64_t>(row) * cols;
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    if constexpr (kOrder == kLanes) {
+                        if (row < rows && column(g, 0) < cols) *reinterpret_cast<Four*>(line + column(g, 0)) = value[j][g];
+                    } else {
+#pragma unroll
+                        for (int t = 0; t < 4; ++t)
+                            if (row < rows && column(g, t) < cols) line[column(g, t)] = value[j][g].v[t];
+                    }
+                }
+            }
+        };
+        batch(std::integral_constant<int, 0>{});
+        if constexpr (kBatch == 2) batch(std::integral_constant<int, 2>{});
+        return;
     }
+    mfma_delta<kOrder>(acc, up, down, rows, cols, rank, row0, col0, lds);
+    const int row = wave_row + n;
+    if (row >= rows) return;
+    const float2 u = row_units<kForm, kExtra>(scale, x, row);
     const int64_t line0 = static_cast<int64_t>(row) * cols;
     if constexpr (kExtra) {
         if (x.more) {
@@ -375,49 +488,36 @@ __global__ __launch_bounds__(kBakeThreads) void bake_kernel(typename Stored<kFor
                     }
         }
     }
-    if constexpr (kForm == kBakeRowwise || kForm == kBakeInt8) {
-        if (!(kExtra && kForm == kBakeRowwise && x.rescale)) over_unit(acc, unit);
-    }
+    if (divides) over_unit(acc, u.x);
     T* const line = data + line0;
     const uint32_t line_at = static_cast<uint32_t>(static_cast<uint64_t>(row) * static_cast<uint64_t>(cols));
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
         const int col = col0 + 64 * g + 16 * q;
-        if constexpr (kVec) {
-            Four four[4];
-            const bool whole = col + 16 <= cols;
-            if (whole) {
+        Four four[4];
+        const bool whole = col + 16 <= cols;
+        if (whole) {
 #pragma unroll
-                for (int t = 0; t < 4; ++t) four[t] = *reinterpret_cast<const Four*>(line + col + 4 * t);
-            } else {
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    if (col + 4 * t < cols) four[t] = *reinterpret_cast<const Four*>(line + col + 4 * t);
-                    else four[t] = Four{};
-            }
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    four[t].v[i] = bake_one<kForm, kExtra>(four[t].v[i], acc[g][t][i], unit, fresh, x,
-                                                           line_at + col + 4 * t + i, seed, k1);
-            if (whole) {
-#pragma unroll
-                for (int t = 0; t < 4; ++t) *reinterpret_cast<Four*>(line + col + 4 * t) = four[t];
-            } else {
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    if (col + 4 * t < cols) *reinterpret_cast<Four*>(line + col + 4 * t) = four[t];
-            }
+            for (int t = 0; t < 4; ++t) four[t] = *reinterpret_cast<const Four*>(line + col + 4 * t);
         } else {
 #pragma unroll
             for (int t = 0; t < 4; ++t)
+                if (col + 4 * t < cols) four[t] = *reinterpret_cast<const Four*>(line + col + 4 * t);
+                else four[t] = Four{};
+        }
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int c = col + 4 * t + i;
-                    if (c < cols)
-                        line[c] = bake_one<kForm, kExtra>(line[c], acc[g][t][i], unit, fresh, x, line_at + c, seed, k1);
-                }
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                four[t].v[i] = bake_one<kForm, kExtra>(four[t].v[i], acc[g][t][i], u.x, u.y, x,
+                                                       line_at + col + 4 * t + i, seed, k1);
+        if (whole) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) *reinterpret_cast<Four*>(line + col + 4 * t) = four[t];
+        } else {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                if (col + 4 * t < cols) *reinterpret_cast<Four*>(line + col + 4 * t) = four[t];
         }
     }
 }
@@ -828,11 +928,12 @@ hipError_t launch_bake(void* data, const float* scale, const float* up, const fl
     const bool vec = cols % 4 == 0 && reinterpret_cast<uintptr_t>(data) % (4 * sizeof(T)) == 0;
     const Extra x{o.gain, o.more, (o.flags & kBakeNearest) != 0, (o.flags & kBakeNoDelta) != 0, o.rescale};
     const bool extra = o.gain || o.more || o.flags || o.rescale;
-#define COZYQ_BAKE(V, E) hipLaunchKernelGGL((bake_kernel<kForm, V, E>), grid, block, 0, s, d, scale, up, down, x, rows, cols, rank, seed)
+#define COZYQ_BAKE(O, E) hipLaunchKernelGGL((bake_kernel<kForm, O, E>), grid, block, 0, s, d, scale, up, down, x, rows, cols, rank, seed)
     if (vec) {
-        if (extra) COZYQ_BAKE(true, true); else COZYQ_BAKE(true, false);
+        constexpr BakeOrder kWhole = sizeof(T) == 1 ? kRuns : kLanes;
+        if (extra) COZYQ_BAKE(kWhole, true); else COZYQ_BAKE(kWhole, false);
     } else {
-        if (extra) COZYQ_BAKE(false, true); else COZYQ_BAKE(false, false);
+        if (extra) COZYQ_BAKE(kColumns, true); else COZYQ_BAKE(kColumns, false);
     }
 #undef COZYQ_BAKE
     return hipGetLastError();

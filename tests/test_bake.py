@@ -744,6 +744,37 @@ def test_gpu_bake_options_bit_exact(form, gain, more, nearest, no_delta):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("form", [ob.BF16, ob.F16, ob.F32, ob.ROWWISE, ob.INT8])
+@pytest.mark.parametrize("cols,skip", [(260, 0), (260, 1), (131, 0), (4, 0), (1, 0), (3, 2), (190, 0)])
+def test_gpu_bake_lane_orders_bit_exact(form, cols, skip):
+    """Each way a tile falls to its lanes (runs of 16 columns for bytes, whole lines for wider
+    elements, element by element for columns off a multiple of four or weights off a group's
+    alignment), with rows and columns past the tile's end, plain and with every extra: the oracle's
+    bits, and nothing written around the weight."""
+    from cozyq import prebuilt
+
+    rows, rank = 75, 7
+    print(f"bake order form={form} cols={cols} skip={skip}", flush=True)
+    data, scale, rng = _stored_for(form, rows, cols, 3 * cols + form)
+    up = (rng.standard_normal((rows, rank)) * 0.1).astype(np.float32)
+    down = (rng.standard_normal((rank, cols)) * 0.1).astype(np.float32)
+    for extra in (False, True):
+        g, m = _extras(rng, rows, cols, extra and form not in (ob.ROWWISE, ob.INT8), extra)
+        with np.errstate(all="ignore"):
+            want = ob.bake(form, data, scale, up, down, 99, gain=g, more=m)
+        t = _torch_data(form, data)
+        around = torch.zeros(skip + t.numel() + 64, dtype=t.dtype)
+        around[skip : skip + t.numel()] = t.reshape(-1)
+        held = around.to(CUDA)
+        view = held[skip : skip + t.numel()].view(rows, cols)
+        assert view.data_ptr() % (4 * view.element_size()) == skip * view.element_size()
+        prebuilt.library(0).bake(form, view, _cuda(scale), _cuda(up), _cuda(down), 99, gain=_cuda(g), more=_cuda(m))
+        assert np.array_equal(_bytes(view.contiguous()), want.view(np.uint8).reshape(rows, -1))
+        held[skip : skip + t.numel()] = 0
+        assert not held.view(torch.uint8).any()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("gain,more,nearest,no_delta", EXTRA)
 def test_gpu_bake_nvfp4_options_bit_exact(gain, more, nearest, no_delta):
     from cozyq import prebuilt
