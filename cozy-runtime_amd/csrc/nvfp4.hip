@@ -190,13 +190,15 @@ __global__ __launch_bounds__(64 * kGemvWaves) void nvfp4_gemv_kernel(const uint1
 // and feeds four MFMAs for each of kCols blocks of 16 activation rows, on the same columns of both
 // (column 128t + 32·(l/16) + 8q .. + 8 for MFMA q, as the GEMV above does). An activation piece
 // serves the kTiles tiles, and so does a scale load: the 16 bytes of a 128x4 tile's row hold the
-// scales of rows 32 apart. Two passes of kSteps steps' loads are in flight. Every load is in bounds
-// by itself: rows past N or M and steps past the wave's last read the last one, and nothing uses
-// what they bring. The waves' partial sums meet in LDS and are added in wave order; a wave's steps
+// scales of rows 32 apart. A pass issues kSteps steps' loads, then works on them; the other waves of
+// the SIMD fill its wait (one set of load registers leaves room for twice the waves two sets did:
+// K=3072 N=12288 M=40 24.1 us with two, 15.2 with one). Every load is in bounds by itself: rows past
+// N or M and steps past the wave's last read the last one, and nothing uses what they bring; a wave
+// without a step issues none. The waves' partial sums meet in LDS and are added in wave order; a wave's steps
 // do not depend on kSteps, kCols or kTiles, so a row's result does not depend on M.
 //
 // Bound: the activation reads through L2 and the loads' latency; the stream alone is 6 us of K=4096
-// N=14336's 11.3 at 5 rows. The decode is not (bf16's, twice the instructions, measures 0.2 us more).
+// N=14336's 10.6 at 5 rows. The decode is not (bf16's, twice the instructions, measures 0.2 us more).
 // fp16 activations decode by v_cvt_scalef32_pk_f16_fp4 and a packed fp16 multiply by the scale, both
 // exact (2 + 4 significant bits, 2^-10 .. 2688): one instruction a weight where the float32 way takes
 // two and a half. bf16 has no packed multiply and keeps it.
@@ -263,9 +265,10 @@ __global__ __launch_bounds__(64 * kTileWaves) void nvfp4_tiles_kernel(
     };
     const int mine = (steps - wave + kTileWaves - 1) / kTileWaves;  // the wave's steps
     auto issue = [&](int first, Loads& f) {
+        if (mine <= 0) return;  // uniform: more waves than steps
 #pragma unroll
         for (int j = 0; j < kSteps; ++j) {
-            const int t = min(wave + kTileWaves * min(first + j, max(mine - 1, 0)), steps - 1);
+            const int t = wave + kTileWaves * min(first + j, mine - 1);
 #pragma unroll
             for (int i = 0; i < kTiles; ++i)
                 f.code[j][i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wr, code_at[i], 64 * t, kTilePolicy));
@@ -313,24 +316,10 @@ __global__ __launch_bounds__(64 * kTileWaves) void nvfp4_tiles_kernel(
     const int passes = (steps + kTileWaves * kSteps - 1) / (kTileWaves * kSteps);
     Loads a;
     issue(0, a);
-    // Two sets of loads where they fit the registers; else the other wave of the SIMD fills the wait.
-    constexpr bool kTwoSets = kSteps * (5 * kTiles + 16 * kCols) <= 72;
-    if (passes == 1) {
-        multiply(0, a);
-    } else if constexpr (!kTwoSets) {
-        multiply(0, a);
-        for (int p = 1; p < passes; ++p) {
-            issue(p * kSteps, a);
-            multiply(p * kSteps, a);
-        }
-    } else {
-        Loads b;
-        for (int p = 0; p < passes; p += 2) {
-            issue((p + 1) * kSteps, b);
-            multiply(p * kSteps, a);
-            issue((p + 2) * kSteps, a);
-            multiply((p + 1) * kSteps, b);
-        }
+    multiply(0, a);
+    for (int p = 1; p < passes; ++p) {
+        issue(p * kSteps, a);
+        multiply(p * kSteps, a);
     }
 
     // D[i][m]: lane holds MFMA rows 4·(lane/16) + 0..3 of column m = lane % 16. Wave b adds block b's
@@ -537,9 +526,10 @@ hipError_t nvfp4_gemv(const void* x, bool x_half, const uint8_t* w, const uint8_
         return out_half ? by_rows(F{}, T{}) : by_rows(F{}, F{});
     }
     // Whole 128-column steps: the row-tile form, as many 16-row tiles a workgroup as leave one
-    // workgroup a CU (us, graph replays over weights past the MALL, K-split or row-block form / this:
-    // K=4096 N=14336 M=5 14.7 / 11.3, M=16 15.4 / 13.7, M=64 29.7 / 24.5; K=3072 N=9216 M=24 24.9 /
-    // 16.0; K=14336 N=4096 M=2 14.9 / 12.7, M=64 73.5 / 60.7). Where a tile a workgroup is all there is
+    // workgroup a CU (us, graph replays over weights past the MALL, K-split form or 64-row blocks over
+    // all of K / this: K=4096 N=14336 M=5 14.5 / 10.6, M=16 15.1 / 12.5, M=40 22.0 / 18.9, M=64 29.1 /
+    // 23.9; K=3072 N=9216 M=24 24.2 / 11.6; K=14336 N=4096 M=2 14.9 / 12.6, M=64 72.2 / 56.3; K=1024
+    // N=3072 M=5 4.0 / 3.4; K=256 N=1024 M=8 2.9 / 2.5). Where a tile a workgroup is all there is
     // (N <= 4096) nothing shares the activation, and 9..48 rows keep the K-split form, the same bits
     // (K=3072 N=3072 M=40 13.3 / 15.8; K=14336 N=4096 M=16 21.1 / 21.5).
     // Scales that don't start at a dword keep the K-split form too, which reads them two bytes at a time.
@@ -550,15 +540,17 @@ hipError_t nvfp4_gemv(const void* x, bool x_half, const uint8_t* w, const uint8_
             hipLaunchKernelGGL(kernel, dim3((N + 127) / 128 * (8 / share)), dim3(64 * kTileWaves), 0, s, xp, w, scale, scale_2, op, out_half, M, N, K);
             return hipGetLastError();
         };
-        // One step a pass, or all of a short K in one (K=4096 N=4096 M=5 6.3 us and 5.7; K=2048 N=6144
-        // M=7 5.9 and 5.1); longer passes of more tiles hold too many registers.
+        // One step a pass, or all of a short K in one (K=4096 N=4096 M=5 6.3 us and 5.6; K=2048 N=6144
+        // M=7 5.9 and 5.1; but no more steps than there are: K=512 N=3072 M=5 5.3 with four, 3.1 with
+        // one), or two of a long one (K=14336 N=4096 M=2 13.1 and 12.6). Longer passes of more tiles
+        // hold too many registers.
         const int steps = K / 128;
         auto by = [&](auto xh) {
             constexpr bool kX = decltype(xh)::value;
             const int cols = (M + 15) / 16;
             if (share == 4) {
                 switch (cols) {
-                    case 1: return tiled(nvfp4_tiles_kernel<kX, 1, 1, 4>);
+                    case 1: return steps >= 64 ? tiled(nvfp4_tiles_kernel<kX, 2, 1, 4>) : tiled(nvfp4_tiles_kernel<kX, 1, 1, 4>);
                     case 2: return tiled(nvfp4_tiles_kernel<kX, 1, 2, 4>);
                     case 3: return tiled(nvfp4_tiles_kernel<kX, 1, 3, 4>);
                     default: return tiled(nvfp4_tiles_kernel<kX, 1, 4, 4>);
@@ -566,13 +558,20 @@ hipError_t nvfp4_gemv(const void* x, bool x_half, const uint8_t* w, const uint8_
             }
             if (share == 2) {
                 switch (cols) {
-                    case 1: return steps <= 16 ? tiled(nvfp4_tiles_kernel<kX, 2, 1, 2>) : tiled(nvfp4_tiles_kernel<kX, 1, 1, 2>);
+                    case 1: return steps > 8 && steps <= 16 ? tiled(nvfp4_tiles_kernel<kX, 2, 1, 2>) : tiled(nvfp4_tiles_kernel<kX, 1, 1, 2>);
                     case 2: return tiled(nvfp4_tiles_kernel<kX, 1, 2, 2>);
                     case 3: return tiled(nvfp4_tiles_kernel<kX, 1, 3, 2>);
                     default: return tiled(nvfp4_tiles_kernel<kX, 1, 4, 2>);
                 }
             }
-            if (cols == 1) return steps <= 32 ? tiled(nvfp4_tiles_kernel<kX, 4, 1, 1>) : tiled(nvfp4_tiles_kernel<kX, 1, 1, 1>);
+            if (cols == 1) {
+                switch ((steps + kTileWaves - 1) / kTileWaves) {
+                    case 2: return tiled(nvfp4_tiles_kernel<kX, 2, 1, 1>);
+                    case 3: return tiled(nvfp4_tiles_kernel<kX, 3, 1, 1>);
+                    case 4: return tiled(nvfp4_tiles_kernel<kX, 4, 1, 1>);
+                    default: return steps >= 64 ? tiled(nvfp4_tiles_kernel<kX, 2, 1, 1>) : tiled(nvfp4_tiles_kernel<kX, 1, 1, 1>);
+                }
+            }
             return tiled(nvfp4_tiles_kernel<kX, 1, 4, 1>);
         };
         return x_half ? by(T{}) : by(F{});

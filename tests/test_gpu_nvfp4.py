@@ -56,11 +56,13 @@ def test_nvfp4_gemv_against_the_exact_product(dtype, m, n, k):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,n,k", [(3, 8, 128), (8, 4096, 4224), (7, 4104, 2048), (5, 4100, 2176), (16, 8192, 128), (17, 8200, 1024),
                                    (33, 5128, 384), (48, 9216, 1152), (64, 12296, 640), (49, 520, 1152), (1, 264, 8192),
-                                   (2, 8328, 4224), (9, 4104, 4096)])  # fmt: skip
+                                   (2, 8328, 4224), (9, 4104, 4096), (4, 264, 1152), (6, 136, 2304), (7, 264, 3968), (8, 1032, 8192),
+                                   (5, 8328, 8320), (3, 4104, 1152), (64, 264, 256)])  # fmt: skip
 def test_nvfp4_row_tiles_against_the_exact_product(dtype, m, n, k):
     """The row-tile kernel at the edges of its dispatch: one, two and four weight tiles a workgroup
-    (256 tiles and one more, 512 and one more), one to four activation blocks, one pass and several
-    with waves that have no step, N off the tile and off a multiple of 4."""
+    (256 tiles and one more, 512 and one more), one to four activation blocks, one pass of one to four
+    steps a wave and several passes of one and of two, with waves that have no step, N off the tile and
+    off a multiple of 4."""
     test_nvfp4_gemv_against_the_exact_product(dtype, m, n, k)
 
 
@@ -88,8 +90,8 @@ def test_nvfp4_gemv_takes_scales_off_their_alignment(m, n, k, skip):
 
 @pytest.mark.parametrize("n,sizes", [(4096, (3, 5, 16, 17, 33, 50)), (12288, (5, 9, 16, 17, 33, 50))])
 def test_nvfp4_gemv_rows_do_not_depend_on_m(n, sizes):
-    """Within a kernel (the streaming form at 1 or 2 rows; the K-split GEMV; the row-block form
-    past 4 rows when N gives 192 64-row groups) a row's bits do not depend on M, and repeat."""
+    """Within a kernel (the streaming form at 1 or 2 rows; the K-split form and the row-tile form, whose
+    sums are the same) a row's bits do not depend on M, and repeat."""
     from cozyq import prebuilt
 
     codes, _, blocked, second, _ = _weight(n, 2048, 9)
