@@ -182,8 +182,9 @@ __device__ __forceinline__ float2 norm_stats(const Prologue& p, const uint16_t* 
 }
 
 
-// Rotation by H_kRot (256: H4^⊗4 then ·1/16; 128: H2⊗H4^⊗3 unnormalized) and per-row int8 of
-// long rows. One block per row; kMaxChunks bounds the row's 4096-element chunks held in registers.
+// Rotation by H_kRot (256: H4^⊗4 then ·1/16; 128: H2⊗H4^⊗3 unnormalized) and per-row int8, by
+// chunks of 4096 elements (`chunked` below says for which rows). One block per row; kMaxChunks bounds
+// the chunks held in registers.
 template <bool kHalf, int kRot, int kMaxChunks, bool kPro = false>
 __global__ __launch_bounds__(kThreads) void rotate_quantize_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ q, float* __restrict__ scales, int K,
@@ -495,19 +496,55 @@ __global__ __launch_bounds__(kThreads) void mx_quantize_kernel(
     if ((i & 3) == 0) scales[i >> 2] = static_cast<uint8_t>(byte);
 }
 
+// Whether rows of K elements run as 4096-element chunks by 4 waves (rotate_quantize_kernel) rather
+// than in one pass by a wave per 1024 (row_block_kernel). At few rows the pass wins (but for the
+// transcendentals of a short row, 16 a thread where the chunks have 8); at many the waves resident on
+// a CU decide, and a pass of 9..11 or 13..16 of them leaves room for too few rows (registers: 24 waves
+// a CU; LDS: one row above ~15600 elements). Each line between both sides' times (us, one pass /
+// chunks): no prologue K=12288 M=512 7.9 / 9.5, M=4096 38.0 / 34.7; K=16384 M=1024 21.8 / 19.0. Layer
+// norm K=14336 M=512 16.7 / 18.8, M=1024 30.3 / 25.9, M=4096 114 / 90; K=9216 M=768 13.7 / 15.6,
+// M=1024 19.6 / 17.8; K=12288 M=4096 65.6 / 66.5. tanh-GELU K=11264 M=1024 20.3 / 22.6, M=4096 75.5 /
+// 67.4; K=6144 M=1024 12.6 / 13.8, M=4096 40.6 / 36.6; K=5120 M=1024 11.2 / 12.6, M=8192 62.3 / 58.8;
+// K=2048 M=16 5.0 / 4.4, M=4096 15.8 / 16.1. [up | gate] rows, twice as long, K=11264 M=4096 87.9 / 87.
+template <bool kPro>
+bool chunked(const Prologue& p, int M, int K, int lds) {
+    if (K > 16 * kBlockMax) return true;
+    const int waves = (K + 1023) / 1024;
+    if (waves == 8) return M > 4096 && p.act == 0;
+    if constexpr (!kPro) return waves > 8 && (M > 1024 || (M > 512 && 2 * lds > 160 * 1024));
+    const bool up_gate = p.act == kActSwiglu && p.up == nullptr;
+    if (waves > 12) return M > (up_gate ? 768 : 512);
+    if (waves == 12) return false;
+    if (waves == 11) return M > 1280 && !up_gate;
+    if (waves > 8) return M > 768;
+    if (waves == 6) return M > 1024;
+    if (p.act == 0) return false;
+    if (waves == 7) return M > 2560;
+    if (waves == 5) return M > 1280;
+    return waves <= 2 && p.norm == 0 && (M <= 1536 || (waves == 2 && K <= 1536));
+}
+
 template <bool kHalf, int kRot, bool kPro>
 hipError_t launch_rotated(const void* x, int8_t* q, float* scales, int M, int K,
                           const Prologue& pro, hipStream_t s) {
     const dim3 grid(M);
     auto xp = static_cast<const uint16_t*>(x);
-    // 9..16 waves a row synchronize too often for many rows: there the 4-wave chunked form streams
-    // better (K=12288 M=4096 38.0 us against 34.7; M=512 7.5 against 9.1).
-    if (!kPro && K > 8192 && K <= 4 * kChunk && M > 1024)
-        rotate_quantize_kernel<kHalf, kRot, 4, kPro><<<grid, kThreads, 0, s>>>(xp, q, scales, K, pro);
-    else if (K <= 16 * kBlockMax)
-        row_block_kernel<kHalf, kRot, kPro><<<grid, 64 * ((K + 1023) / 1024), K / kRot * Layout<kRot>::kGroupStride * 4, s>>>(xp, q, scales, K, pro);
-    else
-        rotate_quantize_kernel<kHalf, kRot, 8, kPro><<<grid, kThreads, 0, s>>>(xp, q, scales, K, pro);
+    const int lds = K / kRot * Layout<kRot>::kGroupStride * 4;
+    if (!chunked<kPro>(pro, M, K, lds)) {
+        row_block_kernel<kHalf, kRot, kPro><<<grid, 64 * ((K + 1023) / 1024), lds, s>>>(xp, q, scales, K, pro);
+        return hipGetLastError();
+    }
+#define COZYQ_CHUNKS(C) rotate_quantize_kernel<kHalf, kRot, C, kPro><<<grid, kThreads, 0, s>>>(xp, q, scales, K, pro)
+    if (K > 4 * kChunk) {
+        COZYQ_CHUNKS(8);
+    } else if (K > 2 * kChunk) {
+        COZYQ_CHUNKS(4);
+    } else if (!kPro || K > kChunk) {
+        COZYQ_CHUNKS(2);
+    } else if constexpr (kPro) {
+        COZYQ_CHUNKS(1);
+    }
+#undef COZYQ_CHUNKS
     return hipGetLastError();
 }
 

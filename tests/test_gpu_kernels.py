@@ -938,6 +938,47 @@ def test_quantize_prologue_within_one_step(ops, fp8, dtype, case):
     assert (got != want).float().mean() <= (0.05 if swiglu else 0.01)
 
 
+#: (rows, K): a partly filled wave, one wave, 4, 5, 9, 12 and 16 waves a row, more than one pass holds;
+#: then both sides of each line at which rows run in chunks.
+PROLOGUE_SHAPES = [(1, 256), (5, 768), (3, 1280), (2, 3840), (1, 5120), (2, 8448), (3, 12288), (2, 16384), (2, 16640),
+                   (1537, 2048), (1537, 1280), (1281, 4352), (1025, 6144), (1024, 6144), (2561, 7168), (769, 9216),
+                   (768, 9216), (1281, 10496), (513, 12544), (769, 12544), (4097, 7424)]  # fmt: skip
+
+
+@pytest.mark.parametrize("shape,case", [(s, c) for s in PROLOGUE_SHAPES for c in PROLOGUES
+                                        if s[0] <= 64 or c[0] not in ("rms", "tables")],
+                         ids=lambda v: v[0] if isinstance(v[0], str) else f"{v[0]}x{v[1]}")  # fmt: skip
+def test_int8_prologue_widths_within_one_step(ops, shape, case):
+    """The int8 quantizer's prologue at the widths its two kernels divide among their lanes: lanes
+    past K must stay out of the norm's sums, which a mean eight deviations from zero shows (each would
+    add 64 variances). The bounds are `test_quantize_prologue_within_one_step`'s."""
+    name, norm, eps, tables, act, with_up = case
+    m, k = shape
+    gated = act == laws.ACT_SITU or (act == laws.ACT_SWIGLU and not with_up)
+    print(f"prologue {name} {m}x{k}", flush=True)
+    x = activations(m, 2 * k if gated else k, seed=m + k)
+    if norm:
+        x = (x.float() + 8.0).to(x.dtype)
+    gen = torch.Generator().manual_seed(k)
+    scale = shift = up = None
+    if tables or name.startswith("layer"):
+        scale = (torch.randn(1, k, generator=gen) * 0.2).to(x.dtype)
+        shift = (torch.randn(1, k, generator=gen) * 0.2).to(x.dtype)
+    if with_up:
+        up = activations(m, k, seed=72)
+    dev = lambda t: None if t is None else t.to(DEV)  # noqa: E731
+    q, s = ops.int8_quantize(x.to(DEV), dev(scale), dev(shift), norm, eps, act, dev(up))
+    rows = sorted({0, m // 2, m - 1})
+    law = laws.prologue(x[rows], scale=scale, shift=shift, norm=norm, eps=eps, activation=act,
+                        up=None if up is None else up[rows])  # fmt: skip
+    wq, ws = laws.quantize_rows_int8(law, 256)
+    got, want, s, ws = q[rows].cpu().float(), wq.float(), s[rows].cpu().reshape(-1, 1), ws.reshape(-1, 1)
+    swiglu = act == laws.ACT_SWIGLU
+    assert ((s - ws).abs() <= (2.0**-7 if swiglu else 1e-5) * ws).all()
+    assert ((got * s - want * ws).abs() <= (2.01 if swiglu else 1.01) * ws + 1e-30).all()
+    assert (got != want).float().mean() <= (0.05 if swiglu else 0.01)
+
+
 # ------------------------------------------------------------------------- w4a8 lane
 
 
