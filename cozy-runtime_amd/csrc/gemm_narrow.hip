@@ -537,6 +537,11 @@ constexpr int kW4MaxK = 8192;    // activation rows a thread stages: K ≤ this
 constexpr int kW4Policy = 3;     // sc0 nt: each code byte is read once per call
 constexpr int kW4RowsMax = 64;   // rows the row-tile form takes (one to four MFMAs' B columns)
 constexpr int kW4RowsK = 1024;   // past 32 rows, with K of this and more
+// Weights of so many 16-row tiles that the narrow tiles fill the chip too keep those past 32 rows
+// (K=4096 M=64 narrow / row tile, us: N=22528 33.2 / 33.2, N=28672 33.7 / 39.1, N=57344 56 / 76), and
+// still wider ones past 16 rows with M·K above 98304 (N=57344 K=4096 M=24 72 / 51, M=32 47 / 53).
+constexpr int kW4RowsTiles = 1536, kW4RowsWide = 2048;
+constexpr int64_t kW4RowsArea = 98304;
 constexpr int kW4GemvRows = 2;   // rows the GEMV form takes
 constexpr uint32_t kFarW4 = 0x7fff0000u;  // a buffer offset past every resource here (reads 0)
 
@@ -731,9 +736,9 @@ __device__ __forceinline__ void int8_store4(i32x4 acc, const Int8Epilogue& e, bo
 // the level table is built); steps past a wave's share read zeros (activation zeros make them
 // add nothing). The waves' int32 partials meet in LDS (exact, in any order), and the epilogue is
 // the int8 law's, so the outputs equal every tile config's bit for bit.
-// Bound: half the time of K=3072 N=12288 M=16 (11.5 us; the 21.2 MB stream alone with everything
+// Bound: a third of the time of K=3072 N=12288 M=16 (9.7 us; the 21.2 MB stream alone with everything
 // else taken out 6.1) is the unpack's VALU work (~90 instructions a step and wave) and the
-// activation reads through L2, neither of which overlaps the one burst of loads. A persistent form
+// activation reads through L2, which overlap only the other workgroup's loads. A persistent form
 // (a workgroup a CU walking its tiles, the next tiles' codes in flight) measured 12.6 - 13.3 there.
 template <int kWaves, int kSteps, int kCols, int kTiles>
 __global__ __launch_bounds__(64 * kWaves) void w4a8_rows_kernel(
@@ -886,34 +891,61 @@ __global__ __launch_bounds__(64 * kWaves) void w4a8_rows_kernel(
     }
 }
 
+// The rows launcher's choices, all of kSteps and kTiles measured against one another (us, graph
+// replays over weights past the MALL).
+// - One step a pass: two or three hold the registers of a second workgroup a CU (K=3072 N=12288 M=16,
+//   three tiles: 11.4 with two steps, 9.7 with one; K=4096 N=8192 M=12 8.5 and 8.2). A weight of at
+//   most 256 tiles leaves the CUs half empty anyway, and takes as few steps in all, dead ones counted,
+//   as 1..4 a pass allow, then the longest passes (K=3072 N=3072 M=3 4.8 with three, 5.1 with one).
+// - Four waves where eight would run out of steps: 9..12 of them (K=1536 N=9216 M=8 6.9 with eight
+//   waves, 6.1 with four) and, at few rows of many tiles, 13..16
+//   (K=2048 N=28672 M=3 12.9 and 11.7).
+// - Tiles a workgroup: a level table and an activation piece serve all of them. Up to 16 rows as many
+//   as leave one workgroup a CU, up to three, and two past that (K=5120 N=14336 M=5 18.7 with four,
+//   16.8 with two). Past 16 rows the partial sums fill the LDS, a
+//   workgroup is alone on its CU, and the rounds over the CUs decide (K=4096 N=17920 M=32 three tiles
+//   23.1, two 26.1; N=28672 M=24 four 28.2, two 31.0).
 template <int kCols>
 hipError_t launch_w4a8_rows(const int8_t* q, const float* xs, const uint8_t* codes, W4 w4, const float* ws,
                             const void* bias, void* out, bool out_half, int M, int N, int K, hipStream_t s) {
     const auto* b = static_cast<const uint16_t*>(bias);
     auto* o = static_cast<uint16_t*>(out);
-    // Steps a wave a pass: as few in all, dead ones counted, as 1 .. 4 a pass allow, then the
-    // longest passes.
-    const int steps = K / 128;
-    int per = 1, least = steps;
-    for (int c = 1; c <= 4; ++c) {
-        const int total = (steps + 8 * c - 1) / (8 * c) * c;
-        if (total <= least) per = c, least = total;
+    const int tiles = (N + 15) / 16, steps = K / 128;
+#define COZYQ_GO(W, S, T) w4a8_rows_kernel<W, S, kCols, T><<<(N + 16 * T - 1) / (16 * T), 64 * W, 0, s>>>(q, xs, codes, w4, ws, b, o, out_half, M, N, K)
+    if constexpr (kCols == 1) {
+        if (steps > 8 && steps <= 12) {
+            if (tiles > 768) COZYQ_GO(4, 3, 2);
+            else COZYQ_GO(4, 3, 1);
+        } else if (M <= 8 && tiles > 1024 && steps > 12 && steps <= 16) {
+            if (tiles > 2048) COZYQ_GO(4, 4, 2);
+            else COZYQ_GO(4, 4, 1);
+        } else if (tiles <= 256) {
+            int per = 1, least = steps;
+            for (int c = 1; c <= 4; ++c) {
+                const int total = (steps + 8 * c - 1) / (8 * c) * c;
+                if (total <= least) per = c, least = total;
+            }
+            if (per == 1) COZYQ_GO(8, 1, 1);
+            else if (per == 2) COZYQ_GO(8, 2, 1);
+            else if (per == 3) COZYQ_GO(8, 3, 1);
+            else COZYQ_GO(8, 4, 1);
+        } else if (tiles > 512 && tiles <= 768) {
+            COZYQ_GO(8, 1, 3);
+        } else {
+            COZYQ_GO(8, 1, 2);
+        }
+    } else {
+        // A round costs its tiles and half a tile's work besides.
+        int share = 1, least = 1 << 30;
+        for (int t = 1; t <= 4; ++t) {
+            const int cost = ((tiles + t - 1) / t + 255) / 256 * (2 * t + 1);
+            if (cost < least) share = t, least = cost;
+        }
+        if (share == 1) COZYQ_GO(8, 1, 1);
+        else if (share == 2) COZYQ_GO(8, 1, 2);
+        else if (share == 3) COZYQ_GO(8, 1, 3);
+        else COZYQ_GO(8, 1, 4);
     }
-    // Tiles a workgroup: as many as leave one workgroup a CU, so that a level table and an
-    // activation piece serve all of a CU's tiles (K=4096 N=14336 M=16 one tile 17.3, four 14.4 us;
-    // M=64 28.0 and 21.0; K=2048 N=8192 M=16 6.6 and 6.0). Up to 8 rows there are few activation
-    // bytes to share and one tile a workgroup, three a CU, is faster (K=3072 N=12288 M=3 10.5
-    // and 9.2), but not past that (K=4096 N=14336 M=5 14.7 and 13.4).
-    const int tiles = (N + 15) / 16;
-    const int share = M <= 8 && tiles <= 768 ? 1 : min(4, (tiles + 255) / 256);
-#define COZYQ_GO(S, T) w4a8_rows_kernel<8, S, kCols, T><<<(N + 16 * T - 1) / (16 * T), 512, 0, s>>>(q, xs, codes, w4, ws, b, o, out_half, M, N, K)
-    if (share == 4) COZYQ_GO(1, 4);
-    else if (share == 3) COZYQ_GO(2, 3);
-    else if (share == 2) COZYQ_GO(2, 2);
-    else if (per == 1) COZYQ_GO(1, 1);
-    else if (per == 2) COZYQ_GO(2, 1);
-    else if (per == 3) COZYQ_GO(3, 1);
-    else COZYQ_GO(4, 1);
 #undef COZYQ_GO
     return hipGetLastError();
 }
@@ -1050,10 +1082,10 @@ hipError_t gemm_w4a8_narrow(const int8_t* q, const float* xs, const uint8_t* cod
     // 1..2 rows by shape: the GEMV form; up to 64 the row-tile kernel (the same bits as every tile
     // config). The GEMV form's MFMA chains grow with the rows, the row tile's do not (graph replays
     // over weights past the MALL, us GEMV / row tile: K=3072 N=12288 M=2 10.2 / 10.0, M=3 13.7 /
-    // 9.1; K=4096 N=14336 M=1 11.2 / 13.3, M=2 12.7 / 13.2). Against the narrow tiles, whose N/64
+    // 8.7; K=4096 N=14336 M=1 11.2 / 13.3, M=2 12.7 / 13.2). Against the narrow tiles, whose N/64
     // workgroups leave the chip idle and run K as one chain (us narrow / row tile): K=12288 N=3072
-    // M=2 64.0 / 11.3, M=16 64.1 / 14.7, M=64 63.6 / 30.9; K=3072 N=12288 M=64 21.7 / 18.3; K=3072
-    // N=3072 M=48 18.5 / 8.5; but K=256 N=14336 M=33 5.5 / 6.5.
+    // M=2 64.0 / 11.3, M=16 64.1 / 14.4, M=64 63.6 / 30.3; K=3072 N=12288 M=64 21.7 / 14.7; K=3072
+    // N=3072 M=48 18.5 / 8.1; but K=256 N=14336 M=33 5.5 / 6.5.
     if (config < 0 && M <= kW4GemvRows && K <= kW4MaxK) {
         const W4 w4{group_scale, codebook};
         if (out_half)
@@ -1063,7 +1095,9 @@ hipError_t gemm_w4a8_narrow(const int8_t* q, const float* xs, const uint8_t* cod
                     : launch_w4a8_decode<false, false>(q, xs, codes, w4, ws, bias, out, M, N, K, s);
     }
     // (A lane's two group scales come in one load, so an odd address keeps the narrow tiles' bytes.)
-    if (config < 0 && M <= kW4RowsMax && (M <= 32 || K >= kW4RowsK) && (reinterpret_cast<uintptr_t>(group_scale) & 1) == 0) {
+    const int tiles = (N + 15) / 16;
+    const bool wide = (M > 32 && tiles > kW4RowsTiles) || (M > 16 && tiles > kW4RowsWide && static_cast<int64_t>(M) * K > kW4RowsArea);
+    if (config < 0 && M <= kW4RowsMax && (M <= 32 || K >= kW4RowsK) && !wide && (reinterpret_cast<uintptr_t>(group_scale) & 1) == 0) {
         const W4 w4{group_scale, codebook};
         switch ((M + 15) / 16) {
             case 1: return launch_w4a8_rows<1>(q, xs, codes, w4, ws, bias, out, out_half, M, N, K, s);

@@ -1043,13 +1043,16 @@ def test_w4a8_linear_bit_exact(ops, shape, codebook):
 @pytest.mark.parametrize("shape", [(2, 136, 12288), (3, 1032, 14336), (16, 264, 12288), (17, 136, 8192),
                                    (33, 136, 4096), (48, 8, 1024), (64, 1032, 12288), (65, 136, 1024),
                                    (20, 4104, 2048), (48, 8200, 1024), (9, 12296, 1024), (64, 14336, 1280),
-                                   (5, 12296, 1280), (8, 9216, 512), (33, 264, 768), (7, 520, 32768)],
+                                   (5, 12296, 1280), (8, 9216, 512), (33, 264, 768), (7, 520, 32768), (3, 264, 1536),
+                                   (16, 12304, 1536), (5, 16400, 2048), (8, 32776, 1792), (17, 16904, 1024),
+                                   (33, 24584, 1024), (64, 18056, 1024), (12, 14344, 2304)],
                          ids=lambda s: "x".join(map(str, s)))  # fmt: skip
 def test_w4a8_row_tiles_bit_exact(ops, shape):
     """The row-tile kernel at the edges of its dispatch: one to four weight tiles a workgroup (256
-    tiles and one more, 512, 768), one to four activation blocks, K in one pass and several with a
-    ragged last one, a last tile of 8 rows, in bf16 and fp16; bit for bit the unpack + int8 GEMM
-    path, and the CPU law on its first rows."""
+    tiles and one more, 512, 768, 1024, 2048), four and eight waves, one to four activation blocks, K
+    in one pass and several with a ragged last one, a last tile of 8 rows, weights wide enough to
+    leave it, in bf16 and fp16; bit for bit the unpack + int8 GEMM path, and the CPU law on its first
+    rows."""
     from cozyq import prebuilt
 
     m, n, k = shape
