@@ -7,7 +7,9 @@
 // A grid of a few hundred tiles runs one round, so its time is one tile's: K/128 steps at what a
 // step costs, and that is the latency of its loads unless several steps are in flight. The two
 // operands come by LDS-DMA in whole 128-byte lines into a ring of kStages steps that fills the CU's
-// LDS (3 to 6 steps, where two co-resident workgroups of the narrow tiles hold 2 each). Waves are
+// LDS (rows x columns: 6 steps of 32x64 to 64x128, 5 of 96x128, 4 of 128x128 and 160x128, 3 of 96x256
+// to 160x256, 2 of 192x256; MX, with its scales, 5 of 32x64 and 2 of 160x256; two co-resident
+// workgroups of the narrow tiles hold 2 each). Waves are
 // 2 (rows) x 4 (columns); the MFMA's A operand is the W tile and its B operand the X tile, so each
 // lane's four results are four consecutive output columns of one row. int8 runs on
 // v_mfma_i32_16x16x64_i8, fp8 and MX on v_mfma_scale_f32_16x16x128_f8f6f4, a step's K in the same
@@ -38,9 +40,14 @@ struct Mid {
     static constexpr int kXGroups = (kTM + 63) / 64;
     static constexpr int kGroups = kKind == kMx ? kXGroups + kTN / 64 : 0;
     static constexpr int fit(int slots) { return (kMidLds - kMidEpi - slots * kGroups * 1024) / kStage; }
-    static constexpr int kStages = fit(3) >= 6 ? 6 : fit(2) > 5 ? 5 : fit(2);
-    static constexpr int kSlots = kStages == 6 ? 3 : 2;
-    static constexpr int kBytes = kStages * kStage + kSlots * kGroups * 1024 + kMidEpi;
+    static constexpr int slots(int stages) { return stages == 6 ? 3 : 2; }
+    static constexpr int bytes(int stages) { return stages * kStage + slots(stages) * kGroups * 1024 + kMidEpi; }
+    static constexpr int kMost = fit(3) >= 6 ? 6 : fit(2) > 5 ? 5 : fit(2);
+    // One step less where it lets a CU hold two (MX 32x64: K=3072 N=9216 M=65 19.9 us with six, 15.7).
+    static constexpr int kStages = kMost == 6 && 2 * bytes(6) > kMidLds && 2 * bytes(5) <= kMidLds ? 5 : kMost;
+    static constexpr int kSlots = slots(kStages);
+    static constexpr int kBytes = bytes(kStages);
+    static constexpr int kHeld = kMidLds / kBytes;  // workgroups a CU's LDS holds
     static constexpr int kBlocks = (kTM + kTN) / 8;    // 8-row loads a step, over 8 waves
     static constexpr int kEach = kBlocks / 8;          // every wave's
     static constexpr int kExtra = kBlocks % 8;         // waves with one more
@@ -333,13 +340,18 @@ hipError_t launch_mid(MidArgs p, hipStream_t s) {
 
 struct MidTile {
     int rows, cols;
-    int each;    // workgroups of it a CU's LDS holds
+    int held;    // workgroups of it a CU holds
     float step;  // us a 128-byte K step
 };
-constexpr MidTile kMidTiles[] = {{32, 64, 2, 0.24f},   {64, 64, 1, 0.23f},  {64, 128, 1, 0.43f},
-                                 {96, 128, 1, 0.50f},  {128, 128, 1, 0.58f}, {160, 128, 1, 0.68f},
-                                 {96, 256, 1, 0.83f},  {128, 256, 1, 0.95f}, {160, 256, 1, 1.15f},
-                                 {192, 256, 1, 1.40f}};
+template <int kTM, int kTN>
+constexpr MidTile mid_tile(float step) {
+    static_assert(Mid<kInt8, kTM, kTN>::kHeld == Mid<kFp8, kTM, kTN>::kHeld && Mid<kInt8, kTM, kTN>::kHeld == Mid<kMx, kTM, kTN>::kHeld, "one table for every kind");
+    return {kTM, kTN, Mid<kInt8, kTM, kTN>::kHeld, step};
+}
+constexpr MidTile kMidTiles[] = {mid_tile<32, 64>(0.24f),  mid_tile<64, 64>(0.23f),   mid_tile<64, 128>(0.43f),
+                                 mid_tile<96, 128>(0.50f), mid_tile<128, 128>(0.58f), mid_tile<160, 128>(0.68f),
+                                 mid_tile<96, 256>(0.83f), mid_tile<128, 256>(0.95f), mid_tile<160, 256>(1.15f),
+                                 mid_tile<192, 256>(1.40f)};
 
 template <int kKind>
 hipError_t mid_by_tile(int tile, const MidArgs& p, hipStream_t s) {
@@ -379,7 +391,7 @@ int mid_choice(int kind, int M, int N, int K) {
     constexpr int kTiles = sizeof(kMidTiles) / sizeof(kMidTiles[0]);
     for (int t = 0; t < kTiles; ++t) {
         const MidTile& m = kMidTiles[t];
-        const float cost = rounds(m.rows, m.cols, kCUs * m.each) * (steps * m.step + kFixed);
+        const float cost = rounds(m.rows, m.cols, kCUs * m.held) * (steps * m.step + kFixed);
         if (best < 0 || cost < least) best = t, least = cost;
     }
     const float tail = tail_columns(M, N) > 0 ? 0.45f : 0.0f;  // its last round runs as half-width tiles

@@ -723,7 +723,7 @@ def test_mid_tiles_bit_equal(ops, shape, dtype):
     assert_close(got[rows], laws.fp8_exact(x[rows], f8, f8s, b))
 
 
-@pytest.mark.parametrize("shape", [(1, 616, 128), (65, 8328, 128), (66, 11024, 384), (131, 11032, 640), (193, 10912, 896),
+@pytest.mark.parametrize("shape", [(1, 616, 128), (65, 8328, 128), (20, 20488, 1152), (66, 11024, 384), (131, 11032, 640), (193, 10912, 896),
                                    (259, 10928, 128), (323, 10920, 256), (386, 13176, 512), (521, 13168, 1152),
                                    (806, 12344, 128), (40, 264, 8192), (300, 1032, 2176)],
                          ids=lambda s: "x".join(map(str, s)))  # fmt: skip
