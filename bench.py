@@ -24,6 +24,7 @@ Prints one JSON line. Only one GPU is used; `--gpus` above 1 exits with a messag
 from __future__ import annotations
 
 import argparse
+import ctypes
 import json
 import os
 import sys
@@ -623,9 +624,11 @@ def bench_svdq_nvfp4(torch, ops, lib, stream, steps: int) -> dict:
 
 
 def bench_tiles(torch, ops, lib, stream, steps: int) -> dict:
-    """The GEMM tile configs (`cozyq_gemm` config 0..5) at the shapes the shape rule
-    (`cozyq_gemm_config`) was fitted on, int8 and fp8, as interleaved medians: each shape's per-
-    config microseconds, the fastest config and the one config -1 runs."""
+    """The GEMM tile configs (`cozyq_gemm` config 0..5) and the shape rule's choice (-1) at the shapes
+    the rule among the configs (`cozyq_gemm_config`) was fitted on, int8 and fp8, as interleaved
+    medians: each shape's microseconds by config, the fastest of the table, the table's config that
+    the rule takes and the tile between the table's that -1 runs instead (`cozyq_gemm_tile`; null
+    where it runs the config, or one of int8's few-row forms)."""
     from cozyq.prebuilt import GEMM_CONFIGS
 
     shapes = [(16, 14336, 4096), (64, 14336, 4096), (128, 14336, 4096), (128, 3072, 3072),
@@ -635,7 +638,8 @@ def bench_tiles(torch, ops, lib, stream, steps: int) -> dict:
               (512, 3072, 3072), (2048, 3072, 3072), (16384, 3072, 3072), (384, 3072, 3072),
               (768, 3072, 3072), (4096, 1280, 5120), (1536, 3072, 3072), (64, 3072, 3072),
               (32, 12288, 3072)]  # fmt: skip
-    configs = range(GEMM_CONFIGS)
+    configs = [*range(GEMM_CONFIGS), -1]
+    size = ctypes.c_int(), ctypes.c_int()
     timer, rows = Timer(torch), []
     for kind in ("int8", "fp8"):
         for m, n, k in shapes:
@@ -656,8 +660,11 @@ def bench_tiles(torch, ops, lib, stream, steps: int) -> dict:
             est = timer.run(fns[0], 3, 1)
             med = timer.interleaved(fns, samples=9, batch=max(2, min(50, int(2.0 / max(est, 1e-3)))))
             us = {c: round(med[c]["ms"] * 1e3, 2) for c in configs}
-            rows.append({"kind": kind, "M": m, "N": n, "K": k, "us": us, "best": min(us, key=us.get),
-                         "chosen": lib.cozyq_gemm_config(int(kind == "fp8"), m, n, k)})  # fmt: skip
+            tile = lib.cozyq_gemm_tile(int(kind == "fp8"), m, n, k, *map(ctypes.byref, size))
+            rows.append({"kind": kind, "M": m, "N": n, "K": k, "us": us,
+                         "best": min(range(GEMM_CONFIGS), key=us.get),
+                         "chosen": lib.cozyq_gemm_config(int(kind == "fp8"), m, n, k),
+                         "tile": None if tile < 0 else f"{size[0].value}x{size[1].value}"})  # fmt: skip
             del q, w
     return {"tiles": rows}
 

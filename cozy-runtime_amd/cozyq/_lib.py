@@ -43,6 +43,9 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
          _P, _P, _P],
     ),
     "cozyq_gemm_config": (c_int, [c_int, c_int, c_int, c_int]),
+    "cozyq_gemm_tile": (
+        c_int, [c_int, c_int, c_int, c_int, ctypes.POINTER(c_int), ctypes.POINTER(c_int)]
+    ),
     "cozyq_svdq_rows": (c_int, [c_int]),
     "cozyq_encode_svdq_int4": (
         c_int, [c_int, _P, c_int, _P, _P, _P, c_int, _P, _P, c_int64, c_int, _P]

@@ -196,6 +196,11 @@ int cozyq_gemm_config(int fp8, int M, int N, int K) {
     return cozyq::gemm_config(fp8 != 0, M, N, K);
 }
 
+int cozyq_gemm_tile(int kind, int M, int N, int K, int* rows, int* cols) {
+    if (kind < 0 || kind > 2 || M < 1 || N < 1 || K < 1 || !rows || !cols) return -1;
+    return cozyq::mid_tile_size(cozyq::mid_choice(kind, M, N, K), rows, cols);
+}
+
 int cozyq_gemm_ex(int device, int fp8, const void* q, const float* scales, const void* w,
                   const float* w_scale, const void* bias, void* out, int64_t ldo, int out_half,
                   int M, int N, int K, int epilogue, void* stream) {

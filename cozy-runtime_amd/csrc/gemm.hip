@@ -128,8 +128,8 @@ hipError_t gemm_int8(const int8_t* q, const float* xs, const int8_t* w, const fl
         const hipError_t e = int8_rows_gemm(q, xs, w, ws, bias, out, ldo, out_half, M, N, K, s);
         if (e != hipErrorNotSupported) return e;
     }
-    if (config < 0 && mid_choice(kInt8, M, N, K) >= 0)
-        return gemm_mid(kInt8, q, xs, nullptr, w, ws, nullptr, bias, out, ldo, out_half, M, N, K, epilogue, s);
+    if (const int tile = config < 0 ? mid_choice(kInt8, M, N, K) : -1; tile >= 0)
+        return gemm_mid(kInt8, tile, q, xs, nullptr, w, ws, nullptr, bias, out, ldo, out_half, M, N, K, epilogue, s);
     if (config < 0) config = gemm_config(false, M, N, K);
     if (config > 0 && config < 5)
         return gemm_int8_narrow(q, xs, w, ws, bias, out, ldo, out_half, M, N, K, epilogue, config, s);
@@ -146,8 +146,8 @@ hipError_t gemm_int8_acc(const int8_t* q, const int8_t* w, int32_t* acc, int M, 
 hipError_t gemm_fp8(const uint8_t* q, const float* xs, const uint8_t* w, const float* ws,
                     const void* bias, void* out, int64_t ldo, bool out_half, int M, int N, int K,
                     int epilogue, int config, hipStream_t s) {
-    if (config < 0 && mid_choice(kFp8, M, N, K) >= 0)
-        return gemm_mid(kFp8, q, xs, nullptr, w, ws, nullptr, bias, out, ldo, out_half, M, N, K, epilogue, s);
+    if (const int tile = config < 0 ? mid_choice(kFp8, M, N, K) : -1; tile >= 0)
+        return gemm_mid(kFp8, tile, q, xs, nullptr, w, ws, nullptr, bias, out, ldo, out_half, M, N, K, epilogue, s);
     if (config < 0) config = gemm_config(true, M, N, K);
     if (config > 0 && config < 5)
         return gemm_fp8_narrow(q, xs, w, ws, bias, out, ldo, out_half, M, N, K, epilogue, config, s);
@@ -158,8 +158,8 @@ hipError_t gemm_fp8(const uint8_t* q, const float* xs, const uint8_t* w, const f
 hipError_t gemm_mx(const uint8_t* q, const uint8_t* qe, const uint8_t* w, const uint8_t* we,
                    const void* bias, void* out, int64_t ldo, bool out_half, int M, int N, int K,
                    hipStream_t s) {
-    if (mid_choice(kMx, M, N, K) >= 0)
-        return gemm_mid(kMx, q, nullptr, qe, w, nullptr, we, bias, out, ldo, out_half, M, N, K, 0, s);
+    if (const int tile = mid_choice(kMx, M, N, K); tile >= 0)
+        return gemm_mid(kMx, tile, q, nullptr, qe, w, nullptr, we, bias, out, ldo, out_half, M, N, K, 0, s);
     return dispatch<kMx>(q, nullptr, w, nullptr, qe, we, bias, out, ldo, out_half, M, N, K, 0,
                          wide_tile(M, N), s);
 }

@@ -373,8 +373,7 @@ hipError_t mid_by_tile(int tile, const MidArgs& p, hipStream_t s) {
 }  // namespace
 
 // The tile for a shape, by a model of the round fitted on MI355X (fp8 and int8, 40 shapes of M 33 to
-// 2048, N 1000 to 14336, K 1280 to 12288; within ~12% of the best tile measured at each): a grid
-// costs its rounds over the CUs, a round kFixed and K/128 steps of what the tile's step costs, which
+// 2048, N 1000 to 14336, K 1280 to 12288; within ~12% of the best tile measured at each): a grid costs its rounds over the CUs, a round kFixed and K/128 steps of what the tile's step costs, which
 // is its LDS traffic (the step's bytes written by DMA and read 1 to 3 times as fragments).
 int mid_choice(int kind, int M, int N, int K) {
     constexpr int64_t kCUs = 256;
@@ -405,10 +404,16 @@ int mid_choice(int kind, int M, int N, int K) {
     return best;
 }
 
-hipError_t gemm_mid(int kind, const void* q, const float* xs, const uint8_t* qe, const void* w,
+int mid_tile_size(int tile, int* rows, int* cols) {
+    if (tile < 0) return -1;
+    *rows = kMidTiles[tile].rows;
+    *cols = kMidTiles[tile].cols;
+    return tile;
+}
+
+hipError_t gemm_mid(int kind, int tile, const void* q, const float* xs, const uint8_t* qe, const void* w,
                     const float* ws, const uint8_t* we, const void* bias, void* out, int64_t ldo,
                     bool out_half, int M, int N, int K, int epilogue, hipStream_t s) {
-    const int tile = mid_choice(kind, M, N, K);
     const MidArgs p{static_cast<const uint8_t*>(q), static_cast<const uint8_t*>(w), xs, ws, qe, we,
                     static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(out), ldo, M, N, K, 0, 0,
                     out_half, epilogue};

@@ -70,10 +70,12 @@ int narrow_config(int M, int N);
 int tail_columns(int M, int N);
 
 // The mid-size tiles (gemm_mid.hip) for kind 0 int8, 1 fp8, 2 MX: the tile their rule takes for a
-// shape (its number, or -1 where the narrow or the 256-row tiles serve), and the GEMM on it. Row
-// scales and epilogue as gemm_int8's / gemm_fp8's; MX takes E8M0 grids qe and we and no epilogue.
+// shape (its number, or -1 where the narrow or the 256-row tiles serve), that tile's rows and columns
+// (and its number), and the GEMM on it. Row scales and epilogue as gemm_int8's / gemm_fp8's; MX takes
+// E8M0 grids qe and we and no epilogue.
 int mid_choice(int kind, int M, int N, int K);
-hipError_t gemm_mid(int kind, const void* q, const float* xs, const uint8_t* qe, const void* w,
+int mid_tile_size(int tile, int* rows, int* cols);
+hipError_t gemm_mid(int kind, int tile, const void* q, const float* xs, const uint8_t* qe, const void* w,
                     const float* ws, const uint8_t* we, const void* bias, void* out, int64_t ldo,
                     bool out_half, int M, int N, int K, int epilogue, hipStream_t s);
 hipError_t gemm_int8(const int8_t* q, const float* xs, const int8_t* w, const float* ws,

@@ -98,10 +98,17 @@ int cozyq_gemm(int device, int family, int fp8, const void* q, const float* scal
                int out_half, int M, int N, int K, int config, cozyq_allocate_fn allocate,
                void* allocate_context, void* stream);
 
-/* The config cozyq_gemm (and cozyq_gemm_ex, which always chooses) runs for config -1 at this
- * shape, where config -1 takes one of the table's tiles (reference: the `choose` of gemm_sm80.cu:283-288 and gemm_fp8.cu:23-29, which the
- * reference does not export); -1 for a non-positive dimension. */
+/* The config of cozyq_gemm's table that the shape rule takes at this shape (reference: the `choose`
+ * of gemm_sm80.cu:283-288 and gemm_fp8.cu:23-29, which the reference does not export); -1 for a
+ * non-positive dimension. Config -1 (and cozyq_gemm_ex, which always chooses) runs it unless
+ * cozyq_gemm_tile names a tile, or one of the few-row int8 forms above serves. */
 int cozyq_gemm_config(int fp8, int M, int N, int K);
+
+/* The tile between the table's narrow and 256-row ones that config -1 runs at this shape on the
+ * current device, for kind 0 int8, 1 fp8 (cozyq_gemm, cozyq_gemm_ex) and 2 MX (cozyq_mx_gemm): its
+ * number from 0 on, its rows and columns in *rows and *cols; -1, and those untouched, where none is
+ * (the MX GEMM then runs a 256-row tile) or for a bad argument. No reference counterpart. */
+int cozyq_gemm_tile(int kind, int M, int N, int K, int* rows, int* cols);
 
 /* cozyq_gemm with an epilogue activation (no reference counterpart: the reference's epilogue
  * is scales + bias only). epilogue 0: none; 1: tanh-GELU applied in float32 to the result of

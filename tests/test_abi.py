@@ -42,13 +42,14 @@ def test_constants():
 
 
 def test_gemm_config_rule():
-    """`cozyq_gemm_config` (what config -1 runs): from 160 256x256 tiles a 256-row tile, the
+    """`cozyq_gemm_config` (the table's config that config -1 runs where no tile between the table's
+    serves, `cozyq_gemm_tile`): from 160 256x256 tiles a 256-row tile, the
     256x192 one (5) where its grid needs fewer than 6/5 the rounds of 256x256 tiles over the 256
     CUs (a round of 3/4-size tiles at ~90% of the rate), else 256x256 (0);
     else, when N gives a 64-column tile 192 workgroups, the one (4: 32x64, 3: 64x64, 2: 128x64)
     that takes every row (up to 128) in one M-tile; else the largest of 1: 128x128, 2: 128x64,
     3: 64x64, 4: 32x64 whose grid reaches 288 workgroups, else 32x64. Each case below is the
-    fastest config the MI355X sweep (`bench.py --only tiles`) measured within 3% at that shape,
+    fastest of the table's configs that the MI355X sweep (`bench.py --only tiles`) measured within 3% at that shape,
     for int8 and fp8 alike, except (8192, 640, 2560), where 128x64 is 8% faster."""
     lib = _lib.load()
     cases = {(4096, 12288, 3072): 0, (4096, 3072, 3072): 5, (1024, 14336, 4096): 0,
@@ -64,6 +65,20 @@ def test_gemm_config_rule():
         for fp8 in (0, 1):
             assert lib.cozyq_gemm_config(fp8, m, n, k) == want, (m, n, k, fp8)
     assert lib.cozyq_gemm_config(0, 0, 8, 256) == -1
+
+
+def test_gemm_tile_names_a_tile_or_none():
+    """`cozyq_gemm_tile`: rows and columns of the tile between the table's, untouched where a table's
+    tile serves and for bad arguments."""
+    lib = _lib.load()
+    rows, cols = ctypes.c_int(-7), ctypes.c_int(-7)
+    at = ctypes.byref(rows), ctypes.byref(cols)
+    for kind, m, n, k in [(0, 128, 3072, 3072), (1, 4096, 3072, 12288), (3, 300, 14336, 4096), (-1, 300, 14336, 4096),
+                          (1, 0, 14336, 4096)]:  # fmt: skip
+        assert lib.cozyq_gemm_tile(kind, m, n, k, *at) == -1 and (rows.value, cols.value) == (-7, -7)
+    assert lib.cozyq_gemm_tile(1, 300, 14336, 4096, at[0], None) == -1
+    assert lib.cozyq_gemm_tile(1, 300, 14336, 4096, *at) >= 0 and (rows.value, cols.value) == (160, 128)
+    assert lib.cozyq_gemm_tile(2, 16, 3072, 3072, *at) >= 0 and (rows.value, cols.value) == (64, 64)
 
 
 def test_nvfp4_entry_points_refuse_bad_shapes_before_the_device():

@@ -689,56 +689,87 @@ def test_every_gemm_config_bit_equal(ops, shape, dtype):
         assert_close(outs[0], laws.fp8_exact(x, f8, f8s, b))
 
 
-#: Shapes the rule gives a mid-size tile, one a tile, with ragged M, N and K among them.
-MID_SHAPES = [(66, 10976, 256), (130, 11152, 256), (193, 10888, 272), (261, 11056, 144), (326, 10896, 256),
-              (385, 13120, 512), (513, 13208, 256), (648, 13128, 144), (200, 3072, 4224), (300, 3080, 5136)]
+def _mid_tile(kind: int, m: int, n: int, k: int) -> tuple[int, int] | None:
+    """The mid-size tile that config -1 runs (`cozyq_gemm_tile`): its rows and columns."""
+    import ctypes
+
+    from cozyq import _lib
+
+    rows, cols = ctypes.c_int(), ctypes.c_int()
+    found = _lib.load().cozyq_gemm_tile(kind, m, n, k, ctypes.byref(rows), ctypes.byref(cols))
+    return (rows.value, cols.value) if found >= 0 else None
+
+
+#: Shapes the rule gives a mid-size tile and that tile, every one of them, with ragged M, N and K.
+MID_SHAPES = [((65, 10248, 4224), (32, 64)), ((200, 3072, 4224), (64, 64)), ((300, 3080, 5136), (64, 64)),
+              ((66, 10976, 256), (64, 128)), ((130, 11152, 256), (96, 128)), ((193, 10888, 272), (128, 128)),
+              ((261, 11056, 144), (160, 128)), ((326, 10896, 256), (96, 256)), ((385, 13120, 512), (128, 256)),
+              ((513, 13208, 256), (160, 256)), ((648, 13128, 144), (192, 256))]  # fmt: skip
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
-@pytest.mark.parametrize("shape", MID_SHAPES, ids=lambda s: "x".join(map(str, s)))
-def test_mid_tiles_bit_equal(ops, shape, dtype):
-    """The shape rule's mid-size tiles: int8 equals the law's product bit for bit (bias, and a
-    strided `out`), fp8 the 256x256 config's bits, with and without bias and tanh-GELU."""
+@pytest.mark.parametrize("shape,tile", MID_SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_mid_tiles_bit_equal(ops, shape, tile, dtype):
+    """The shape rule's mid-size tiles: int8 equals the law's product bit for bit, fp8 the 256x256
+    config's bits, each with and without bias and into a strided `out`; both with tanh-GELU, with and
+    without bias, the law's GELU of that."""
+    from cozyq import prebuilt
+
     m, n, k = shape
+    assert _mid_tile(0, m, n, k) == _mid_tile(1, m, n, k) == tile
     x = activations(m, k, seed=m * 5 + k)
     data, scale = laws.int8_weight_rowwise(weights(n, k, seed=n))
     b = (torch.randn(n, generator=torch.Generator().manual_seed(n)) * 0.1).to(dtype)
     q, s = ops.int8_quantize_rot(x.to(DEV), 0)
+    f8, f8s = laws.fp8_weight(weights(n, k, seed=n + 1))
+    q8, s8 = ops.fp8_quantize(x.to(DEV))
+    w8, w8s = f8.to(DEV), f8s.to(DEV)
     rows = sorted({0, 1, m // 2, m - 17, m - 1})
     for bias in (None, b):
+        dev = None if bias is None else bias.to(DEV)
         want = laws.int8_product(q.cpu()[rows], s.cpu()[rows], data, scale, dtype)
         want = want if bias is None else want + bias
         wide = torch.full((m, n + 64), 7.0, dtype=dtype, device=DEV)
-        dev = None if bias is None else bias.to(DEV)
         got = ops.int8_gemm_ex(q, s, data.to(DEV), scale.to(DEV), dev, dtype, out=wide[:, :n])
         assert torch.equal(got[rows].cpu(), want)
         assert bool((wide[:, n:] == 7.0).all())
-    gelu = ops.int8_gemm_ex(q, s, data.to(DEV), scale.to(DEV), b.to(DEV), dtype, epilogue=1)
-    assert_close(gelu[rows], laws.gelu_tanh(want.float()).double())
-    f8, f8s = laws.fp8_weight(weights(n, k, seed=n + 1))
-    q8, s8 = ops.fp8_quantize(x.to(DEV))
-    for bias in (None, b.to(DEV)):
-        got = ops.fp8_gemm(q8, s8, f8.to(DEV), f8s.to(DEV), bias, dtype)
-        assert torch.equal(got, ops.fp8_gemm(q8, s8, f8.to(DEV), f8s.to(DEV), bias, dtype, 0))
-    assert_close(got[rows], laws.fp8_exact(x[rows], f8, f8s, b))
+        gelu = ops.int8_gemm_ex(q, s, data.to(DEV), scale.to(DEV), dev, dtype, epilogue=1)
+        assert_close(gelu[rows], laws.gelu_tanh(want.float()).double())
+        wide.fill_(7.0)
+        got = ops.fp8_gemm(q8, s8, w8, w8s, dev, dtype, out=wide[:, :n])
+        assert torch.equal(got, ops.fp8_gemm(q8, s8, w8, w8s, dev, dtype, 0))
+        assert bool((wide[:, n:] == 7.0).all())
+        exact = laws.fp8_exact(x[rows], f8, f8s, bias)
+        assert_close(got[rows], exact)
+        gelu = ops._gemm(prebuilt.FP8, q8, s8, w8, w8s, dev, dtype, -1, None, 1)
+        assert_close(gelu[rows], laws.gelu_tanh(exact.float()).double())
 
 
-@pytest.mark.parametrize("shape", [(1, 616, 128), (65, 8328, 128), (20, 20488, 1152), (66, 11024, 384), (131, 11032, 640), (193, 10912, 896),
-                                   (259, 10928, 128), (323, 10920, 256), (386, 13176, 512), (521, 13168, 1152),
-                                   (806, 12344, 128), (40, 264, 8192), (300, 1032, 2176)],
-                         ids=lambda s: "x".join(map(str, s)))  # fmt: skip
-def test_mx_mid_tiles(ops, shape):
+#: MX shapes and the mid-size tile the rule gives each, every one of them.
+MX_MID_SHAPES = [((1, 616, 128), (64, 64)), ((65, 8328, 128), (32, 64)), ((20, 20488, 1152), (32, 64)),
+                 ((66, 11024, 384), (64, 128)), ((131, 11032, 640), (96, 128)), ((193, 10912, 896), (128, 128)),
+                 ((259, 10928, 128), (160, 128)), ((323, 10920, 256), (96, 256)), ((386, 13176, 512), (128, 256)),
+                 ((521, 13168, 1152), (160, 256)), ((806, 12344, 128), (192, 256)), ((40, 264, 8192), (64, 64)),
+                 ((300, 1032, 2176), (64, 64))]  # fmt: skip
+
+
+@pytest.mark.parametrize("shape,tile", MX_MID_SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_mx_mid_tiles(ops, shape, tile):
     """The MX GEMM on the rule's mid-size tiles (one to sixty-four K steps, scale blocks of four
-    steps whole and ragged) against the float64 product of the law's codes, with and without bias."""
+    steps whole and ragged) against the float64 product of the law's codes: bf16 without bias, with
+    one, and fp16 with one."""
     m, n, k = shape
+    assert _mid_tile(2, m, n, k) == tile
     x = activations(m, k, seed=m + k)
     x[:, : k // 2] *= 300.0  # block scales far apart within a row
+    x = x / 64  # fp16 results in range
     data, wscales = laws.mx_quantize(weights(n, k, seed=n))
     q, qs = ops.mx_quantize(x.to(DEV))
     rows = sorted({0, m // 3, max(m - 17, 0), m - 1})
-    b = torch.randn(n, generator=torch.Generator().manual_seed(n)).to(torch.bfloat16)
-    for bias in (None, b):
-        got = ops.mx_gemm(q, qs, data.to(DEV), wscales.to(DEV), None if bias is None else bias.to(DEV), torch.bfloat16)
+    b = torch.randn(n, generator=torch.Generator().manual_seed(n))
+    for bias, dtype in ((None, torch.bfloat16), (b, torch.bfloat16), (b, torch.float16)):
+        bias = None if bias is None else bias.to(dtype)
+        got = ops.mx_gemm(q, qs, data.to(DEV), wscales.to(DEV), None if bias is None else bias.to(DEV), dtype)
         assert_close(got[rows], laws.mx_exact(x[rows], data, wscales, bias))
 
 
