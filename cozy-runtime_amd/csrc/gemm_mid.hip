@@ -373,7 +373,9 @@ hipError_t mid_by_tile(int tile, const MidArgs& p, hipStream_t s) {
 }  // namespace
 
 // The tile for a shape, by a model of the round fitted on MI355X (fp8 and int8, 40 shapes of M 33 to
-// 2048, N 1000 to 14336, K 1280 to 12288; within ~12% of the best tile measured at each): a grid costs its rounds over the CUs, a round kFixed and K/128 steps of what the tile's step costs, which
+// 2048, N 1000 to 14336, K 1280 to 12288; within ~12% of the best tile measured at each; against the
+// narrow and 256-row tiles at 4284 points of M 5 to 3072, N 640 to 128256, K 1024 to 12288 its choices
+// take 0.81 of their time on average and 1.1 at worst): a grid costs its rounds over the CUs, a round kFixed and K/128 steps of what the tile's step costs, which
 // is its LDS traffic (the step's bytes written by DMA and read 1 to 3 times as fragments).
 int mid_choice(int kind, int M, int N, int K) {
     constexpr int64_t kCUs = 256;
@@ -401,6 +403,25 @@ int mid_choice(int kind, int M, int N, int K) {
     // round (K=3072 N=3072 M=77 8.5 us there and 9.0 here; K=12288 N=3072 M=48 23.7 and 29.7; but
     // M=200 39.9 and 28.3). MX has no narrow tiles.
     if (kind != kMx && kMidTiles[best].cols == 64 && (steps <= 32 || rounds(32, 64, kCUs) <= 1.0f)) return -1;
+    if (kind == kMx) return best;
+    const int config = gemm_config(kind == kFp8, M, N, K);
+    if (config == 0 || config == 5) {
+        // At short K and in several rounds what a round costs besides its steps decides: 2.6 us and a
+        // tile's epilogue here, 7 there (fp8 N=12288 M=3072 K=1024 52 us on 256x192, 62 on 192x256).
+        const MidTile& m = kMidTiles[best];
+        const float times = rounds(m.rows, m.cols, kCUs * m.held);
+        const float mid = times * (steps * m.step * m.held + 2.6f + 1.85e-4f * m.rows * m.cols);
+        const float whole = config == 0 ? (rounds(256, 256, kCUs) - tail) * (steps * 1.58f + 7.0f) + 3.0f
+                                        : rounds(256, 192, kCUs) * (steps * 1.38f + 6.5f) + 3.5f;
+        if ((times > 1.0f || steps <= 8) && mid > 0.98f * whole) return -1;
+    } else if (config >= 3 && N <= 3072 && (N + 63) / 64 % 8 == 0) {
+        // A grid of hardly more narrow tiles than CUs, many M-tiles to each XCD's few weight panels,
+        // runs at one tile's pace, 0.3 us a step of 64x64 and 0.22 of 32x64 (K=8192, us, mid / narrow:
+        // M=384 N=3072 30.1 / 25.7, M=768 N=1536 27.5 / 23.1, M=192 N=3072 26.3 / 23.9; past the line
+        // M=416 N=3072 31.5 / 36.2, M=768 N=2048 31.5 / 35.8).
+        const float narrow = rounds(config == 3 ? 64 : 32, 64, 1);
+        if (narrow >= 256.0f && narrow <= (N <= 1536 ? 336.0f : 320.0f)) return -1;
+    }
     return best;
 }
 

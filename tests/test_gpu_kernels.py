@@ -745,6 +745,19 @@ def test_mid_tiles_bit_equal(ops, shape, tile, dtype):
         assert_close(gelu[rows], laws.gelu_tanh(exact.float()).double())
 
 
+def test_mid_tiles_leave_the_narrow_and_the_large_tiles_their_shapes():
+    """Shapes on each side of the lines at which the rule goes back to the narrow tiles (hardly more
+    of them than CUs, on few weight panels; the smallest tiles at short K) and to the 256-row ones."""
+    for kind in (0, 1):
+        for m, n, k in [(384, 3072, 3072), (352, 3072, 8192), (768, 1536, 4096), (896, 1536, 8192), (640, 2048, 4096),
+                        (1280, 1024, 8192), (192, 3072, 8192), (320, 2048, 12288), (64, 3072, 12288), (128, 3072, 3072),
+                        (3072, 12288, 1024), (3072, 7168, 1024), (4096, 12288, 3072), (4096, 3072, 12288)]:  # fmt: skip
+            assert _mid_tile(kind, m, n, k) is None, (kind, m, n, k)
+        for m, n, k in [(416, 3072, 8192), (768, 2048, 8192), (960, 1536, 8192), (224, 3072, 8192), (300, 14336, 4096),
+                        (1024, 9216, 3072), (3072, 3072, 3072), (1179, 9216, 3072)]:  # fmt: skip
+            assert _mid_tile(kind, m, n, k) is not None, (kind, m, n, k)
+
+
 #: MX shapes and the mid-size tile the rule gives each, every one of them.
 MX_MID_SHAPES = [((1, 616, 128), (64, 64)), ((65, 8328, 128), (32, 64)), ((20, 20488, 1152), (32, 64)),
                  ((66, 11024, 384), (64, 128)), ((131, 11032, 640), (96, 128)), ((193, 10912, 896), (128, 128)),
