@@ -347,14 +347,13 @@ __global__ __launch_bounds__(kBlockMax) void row_block_kernel(
 }
 
 // Unrotated rows of at most kRowMaxK elements with no prologue: one wave per row (rows.h), no
-// workgroup barrier, and each wave's next row loaded while it rotates and quantizes the current one, so a
-// CU keeps ~12 rows (72 KB at K = 3072) of loads in flight.
+// workgroup barrier, and each wave's next row loaded while it quantizes the current one, so a CU
+// keeps ~12 rows (72 KB at K = 3072) of loads in flight.
 constexpr int kRowWaves = 4;
 
-template <bool kHalf, int kRot>
+template <bool kHalf>
 __global__ __launch_bounds__(64 * kRowWaves) void row_quantize_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ q, float* __restrict__ scales, int M, int K) {
-    __shared__ __attribute__((aligned(16))) float lds[kRowWaves][kRowLdsFloats<kRot> > 0 ? kRowLdsFloats<kRot> : 1];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int stride = gridDim.x * kRowWaves;
     int row = blockIdx.x * kRowWaves + wave;
@@ -366,11 +365,11 @@ __global__ __launch_bounds__(64 * kRowWaves) void row_quantize_kernel(
     // row, so the loads stay branch-free) are issued before the current row is worked on.
     while (true) {
         row_loads(view(row + stride), lane, b);
-        quantize_row_wave<kHalf, kRot>(a, K, lane, lds[wave], q + static_cast<int64_t>(row) * K, scales + row);
+        quantize_row_wave<kHalf, 0>(a, K, lane, nullptr, q + static_cast<int64_t>(row) * K, scales + row);
         row += stride;
         if (row >= M) break;
         row_loads(view(row + stride), lane, a);
-        quantize_row_wave<kHalf, kRot>(b, K, lane, lds[wave], q + static_cast<int64_t>(row) * K, scales + row);
+        quantize_row_wave<kHalf, 0>(b, K, lane, nullptr, q + static_cast<int64_t>(row) * K, scales + row);
         row += stride;
         if (row >= M) break;
     }
@@ -580,8 +579,8 @@ hipError_t rotate_quantize(const void* x, bool x_half, int8_t* q, float* scales,
         // 12 waves a CU: three 4-wave blocks on each of the 256 CUs, grid-strided over the rows.
         const int blocks = min((M + kRowWaves - 1) / kRowWaves, 3 * 256);
         auto xp = static_cast<const uint16_t*>(x);
-        if (x_half) row_quantize_kernel<true, 0><<<blocks, 64 * kRowWaves, 0, s>>>(xp, q, scales, M, K);
-        else row_quantize_kernel<false, 0><<<blocks, 64 * kRowWaves, 0, s>>>(xp, q, scales, M, K);
+        if (x_half) row_quantize_kernel<true><<<blocks, 64 * kRowWaves, 0, s>>>(xp, q, scales, M, K);
+        else row_quantize_kernel<false><<<blocks, 64 * kRowWaves, 0, s>>>(xp, q, scales, M, K);
         return hipGetLastError();
     }
     if (rotation == 0) {
