@@ -15,8 +15,10 @@
 // v_mfma_i32_16x16x64_i8, fp8 and MX on v_mfma_scale_f32_16x16x128_f8f6f4, a step's K in the same
 // order as the narrow tiles', so int8 and fp8 outputs are theirs bit for bit.
 //
-// Bound: the LDS, written by DMA and read as fragments at ~50 KB a us and CU whatever the tile
-// (compute alone 0.75 us of 128x256's 0.95 us step, DMA alone 0.5 from L2 and 0.9 with W from HBM).
+// Bound: the step. Its bytes go into the LDS and its fragments come out at ~50 KB a us and CU whatever
+// the tile (compute alone 0.75 us of 128x256's 0.95 us step, DMA alone 0.5 from L2 and 0.9 with W from
+// HBM), and no unit is full: at int8 1179x9216x3072 and fp8 300x14336x4096 the MFMAs are busy 45 and
+// 34% of the time, fragment reads 20 and 25% without a bank conflict, and a wave waits 40% of its life.
 // Measured against the narrow and 256-row tiles (us, graph replays over weights past the MALL,
 // before / after): fp8 M=300 N=14336 K=4096 39.9 / 27.7, M=1024 N=9216 K=3072 68.6 / 37.7, M=1500
 // N=3072 K=12288 92.1 / 66.5, M=3072 N=3072 K=3072 58.5 / 37.2; int8 M=642 N=7688 K=3840 39.4 /
@@ -374,9 +376,10 @@ hipError_t mid_by_tile(int tile, const MidArgs& p, hipStream_t s) {
 
 // The tile for a shape, by a model of the round fitted on MI355X (fp8 and int8, 40 shapes of M 33 to
 // 2048, N 1000 to 14336, K 1280 to 12288; within ~12% of the best tile measured at each; against the
-// narrow and 256-row tiles at 4284 points of M 5 to 3072, N 640 to 128256, K 1024 to 12288 its choices
-// take 0.81 of their time on average and 1.1 at worst): a grid costs its rounds over the CUs, a round kFixed and K/128 steps of what the tile's step costs, which
-// is its LDS traffic (the step's bytes written by DMA and read 1 to 3 times as fragments).
+// narrow and 256-row tiles at 7434 points of M 1 to 3072, N 640 to 128256, K 1024 to 12288 its choices
+// take 0.88 of their time on average and 1.09 at worst): a grid costs its rounds over the CUs, a round
+// kFixed and K/128 steps of what the tile's step costs, which is its LDS traffic (the step's bytes
+// written by DMA and read 1 to 3 times as fragments).
 int mid_choice(int kind, int M, int N, int K) {
     constexpr int64_t kCUs = 256;
     constexpr float kFixed = 5.0f;  // us: launch, first loads, epilogue

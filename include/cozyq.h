@@ -169,9 +169,11 @@ int cozyq_gemm_i32(int device, const int8_t* q, const int8_t* w, int32_t* acc, i
  * (internal/prebuilt.py:471-492). The codes are unpacked in registers on the way to the int8
  * MFMA; the epilogue is cozyq_gemm's int8 law with w_scale [N], bit for bit. out [M, N].
  * N % 8 == 0, K % 256 == 0; q and w 16-byte aligned, out 8-byte aligned. config names
- * cozyq_gemm's narrow tiles 1..4 (-1: by rows, a GEMV form for 1..2 rows with K <= 8192 and a
- * row-tile kernel up to 32 rows, 64 with K >= 1024, the same bits); 0 and 5 (the 256-row tiles, which multiply
- * the codes unpacked by cozyq_w4a8_unpack) and 6 and above return hipErrorNotSupported. */
+ * cozyq_gemm's narrow tiles 1..4 (-1: by shape, a GEMV form for 1..2 rows with K <= 8192 and a
+ * row-tile kernel up to 32 rows, 64 with K >= 1024, where s is 2-byte aligned and N is not so
+ * wide that the narrow tiles fill the chip as well: N <= 24576 past 32 rows, N <= 32768 or
+ * M*K <= 98304 past 16; the same bits); 0 and 5 (the 256-row tiles, which multiply the codes
+ * unpacked by cozyq_w4a8_unpack) and 6 and above return hipErrorNotSupported. */
 int cozyq_w4a8_gemm(int device, const int8_t* q, const float* scales, const uint8_t* w,
                     const uint8_t* s, const float* codebook, const float* w_scale, const void* bias,
                     void* out, int out_half, int M, int N, int K, int config, void* stream);
