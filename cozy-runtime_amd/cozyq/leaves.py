@@ -99,13 +99,16 @@ def _read_parts(leaf: Any) -> tuple[Tensor, Tensor, Tensor | None]:
     buffer is found by a miss (1.7 us for the three, 0.2 from the buffers' table, of a call of 13), so a
     leaf of the plain class reads its buffers by name where nothing else holds one of the names: a
     parameter, a parametrization, a property or an attribute of its own."""
-    if type(leaf) is _module_class._cached:
-        own = leaf.__dict__
+    own = leaf.__dict__
+    if type(leaf) is _module_class._cached and not ("data" in own or "scale" in own or "bias" in own):
         held = own["_buffers"]
-        if ("data" in held and "scale" in held and "bias" in held
-                and "data" not in own and "scale" not in own and "bias" not in own):  # fmt: skip
-            return read(held["data"]), read(held["scale"]), read(held["bias"])
-    return read(leaf.data), read(leaf.scale), read(leaf.bias)
+        try:
+            data, scale, bias = held["data"], held["scale"], held["bias"]
+        except KeyError:
+            data, scale, bias = leaf.data, leaf.scale, leaf.bias
+    else:
+        data, scale, bias = leaf.data, leaf.scale, leaf.bias
+    return read(data), read(scale), read(bias)
 
 
 class _QuantizedLane(_Lane):
@@ -126,10 +129,12 @@ class _QuantizedLane(_Lane):
         return int8_linear.quantize(torch, x)
 
     def gemm(self, torch, leaf, operand, out_dtype, out):
-        return int8_linear.gemm(torch, operand, *_read_parts(leaf), out_dtype, out)
+        data, scale, bias = _read_parts(leaf)
+        return int8_linear.gemm(torch, operand, data, scale, bias, out_dtype, out)
 
     def linear(self, torch, leaf, x, out_dtype):
-        return int8_linear.linear(torch, x, *_read_parts(leaf), out_dtype)
+        data, scale, bias = _read_parts(leaf)
+        return int8_linear.linear(torch, x, data, scale, bias, out_dtype)
 
     def run(self, torch, leaf, x, prequantized, out):
         if isinstance(x, PreQuantized):
@@ -154,10 +159,12 @@ class _Fp8Lane(_QuantizedLane):
         return fp8_linear.quantize(torch, x)
 
     def gemm(self, torch, leaf, operand, out_dtype, out):
-        return fp8_linear.gemm(torch, operand, *_read_parts(leaf), out_dtype, out)
+        data, scale, bias = _read_parts(leaf)
+        return fp8_linear.gemm(torch, operand, data, scale, bias, out_dtype, out)
 
     def linear(self, torch, leaf, x, out_dtype):
-        return fp8_linear.linear(torch, x, *_read_parts(leaf), out_dtype)
+        data, scale, bias = _read_parts(leaf)
+        return fp8_linear.linear(torch, x, data, scale, bias, out_dtype)
 
 
 class _W4a8Lane(_QuantizedLane):
